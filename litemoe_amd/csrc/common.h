@@ -129,6 +129,14 @@ __device__ __forceinline__ void lds_copy16(const void *base, uint32_t voff, uint
 // Wait until every vector memory operation this wave issued has completed
 // (s_waitcnt vmcnt(0)), LDS copies included.
 __device__ __forceinline__ void lds_copy_wait() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+// Wait until at most N of this wave's vector memory operations are in flight
+// (they complete in issue order): gfx9's s_waitcnt encoding, vmcnt in bits
+// 3:0 and 15:14, expcnt and lgkmcnt left at their maxima.
+template <int N>
+__device__ __forceinline__ void vm_wait() {
+  static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
+}
 // The 32-bit LDS address of a __shared__ pointer.
 __device__ __forceinline__ uint32_t lds_address(const void *p) {
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char *)p;

@@ -13,12 +13,13 @@
 // eager or replayed from a graph (no split-K partials, no atomics, no stream-K
 // fix-up whose summation order the caller cannot see).
 //
-// Workgroup = kTM x kTN output tile (256 x 256 on 16 waves, or 128 x 128 on
-// 4), kWM x kWN waves, each wave a (kTM/kWM) x (kTN/kWN) block of 16 x 16
-// MFMA tiles; K runs in steps of 64.
-// The next step's A and B rows are copied from global memory straight into
-// the other of two LDS stages (global_load_lds_dwordx4, no register staging)
-// while the MFMAs run on the current step's stage; one barrier per step. An
+// Workgroup = kTM x kTN output tile (16 x 64 to 256 x 256, launch_gemm_tiled),
+// kWM x kWN waves, each wave a (kTM/kWM) x (kTN/kWN) block of 16 x 16 MFMA
+// tiles; K runs in steps of 64.
+// The next steps' A and B rows are copied from global memory straight into
+// the other LDS stages (two to four; global_load_lds_dwordx4, no register
+// staging) while the MFMAs run on the current step's stage; one barrier per
+// step. An
 // LDS row is 64 bf16 = 8 chunks of 16 bytes; chunk c of tile row r sits at
 // position c ^ (r & 7), so the 16 rows of one fragment read spread over the
 // banks, and each copy instruction fills 1 KB contiguously. At the cfg 4 QKV
@@ -77,7 +78,7 @@ __device__ __forceinline__ void rotate3(float x1, float x2, float c, float s, fl
 // out 16-byte aligned), 1 = 8-byte fragment words (N % 4 == 0, ldo % 4 == 0,
 // out 8-byte aligned), 0 = 2-byte stores.
 // kRope: the RopeKV epilogue (64-column wave blocks, kStore >= 1).
-template <int kTM, int kTN, int kWM, int kWN, int kStore, bool kRope = false>
+template <int kTM, int kTN, int kWM, int kWN, int kStages, int kStore, bool kRope = false>
 __global__ void __launch_bounds__(64 * kWM * kWN)
 gemm_kernel(const bf16 *__restrict__ a, int64_t lda, const bf16 *__restrict__ w, int64_t ldw,
             bf16 *__restrict__ out, int64_t ldo, int M, int N, int K, int tiles_m, int tiles_n,
@@ -88,8 +89,10 @@ gemm_kernel(const bf16 *__restrict__ a, int64_t lda, const bf16 *__restrict__ w,
   constexpr int kLA = kTM / (8 * kWaves), kLB = kTN / (8 * kWaves);  // 16-byte loads per lane
   static_assert(kLA * 8 * kWaves == kTM && kLB * 8 * kWaves == kTN, "tile rows per load round");
   constexpr int kABytes = kTM * kRowBytes, kStage = (kTM + kTN) * kRowBytes;
-  __shared__ __align__(16) char s0[kStage];  // two LDS stages
-  __shared__ __align__(16) char s1[kStage];
+  // Two stages are two arrays (as one, the 256 x 256 rope kernel takes four
+  // registers more and 2% more time); three or more are one array.
+  __shared__ __align__(16) char s0[kStages == 2 ? kStage : kStages * kStage];
+  __shared__ __align__(16) char s1[kStages == 2 ? kStage : 16];
   __shared__ int64_t st_pos[kRope ? kTM : 1];  // kRope, kStore == 2: cache position per row
   __shared__ int st_slot[kRope ? kTM : 1];
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
@@ -185,19 +188,44 @@ gemm_kernel(const bf16 *__restrict__ a, int64_t lda, const bf16 *__restrict__ w,
   }
 
   const int nk = K / kBK;
-  issue(0, s0);
-  for (int kt = 0; kt < nk; kt += 2) {
-    lds_copy_wait();
-    __syncthreads();
-    if (kt + 1 < nk) issue(kt + 1, s1);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(s0);
-    if (kt + 1 < nk) {
+  if constexpr (kStages == 2) {
+    issue(0, s0);
+    for (int kt = 0; kt < nk; kt += 2) {
       lds_copy_wait();
       __syncthreads();
-      if (kt + 2 < nk) issue(kt + 2, s0);
+      if (kt + 1 < nk) issue(kt + 1, s1);
       __builtin_amdgcn_sched_barrier(0);
-      compute(s1);
+      compute(s0);
+      if (kt + 1 < nk) {
+        lds_copy_wait();
+        __syncthreads();
+        if (kt + 2 < nk) issue(kt + 2, s0);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(s1);
+      }
+    }
+  } else {
+    // A ring: the copies of kStages - 1 steps are in flight; a step waits for
+    // its own only (they complete in issue order), and one barrier tells that
+    // every wave's copies have landed and that every wave has left the step
+    // whose slot the next copy goes into.
+    static_assert(kStages <= 4, "the waits below leave at most two later steps in flight");
+    constexpr int kL = kLA + kLB;  // copies of one step per wave
+#pragma unroll
+    for (int s = 0; s < kStages - 1; ++s)
+      if (s < nk) issue(s, s0 + s * kStage);
+    int cur = 0, nxt = (kStages - 1) * kStage;
+    for (int kt = 0; kt < nk; ++kt) {
+      const int later = min(nk - 1 - kt, kStages - 2);  // steps in flight behind this one
+      if (later == 0) vm_wait<0>();
+      else if (later == 1) vm_wait<kL>();
+      else vm_wait<2 * kL>();
+      __syncthreads();
+      if (kt + kStages - 1 < nk) issue(kt + kStages - 1, s0 + nxt);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(s0 + cur);
+      cur = cur == (kStages - 1) * kStage ? 0 : cur + kStage;
+      nxt = nxt == (kStages - 1) * kStage ? 0 : nxt + kStage;
     }
   }
 
@@ -239,8 +267,8 @@ gemm_kernel(const bf16 *__restrict__ a, int64_t lda, const bf16 *__restrict__ w,
     // Staged row r's 16-byte chunk c sits at c ^ (r & kSw): the 16 rows of
     // one fragment store fall on different bank groups.
     constexpr int kOB = kTN * 2, kChunks = kOB / 16, kSw = (kChunks < 16 ? kChunks : 16) - 1;
-    constexpr int kHalfRows = kStage / kOB;  // rows held by the first stage
-    static_assert(kTM * kOB <= 2 * kStage, "output tile fits the LDS stages");
+    constexpr int kHalfRows = (kStages == 2 ? kStage : kStages * kStage) / kOB;  // rows held by s0
+    static_assert(kTM * kOB <= kStages * kStage, "output tile fits the LDS stages");
     auto staged = [&](int r) -> char * {
       if constexpr (kTM <= kHalfRows) return s0 + r * kOB;
       else return r < kHalfRows ? s0 + r * kOB : s1 + (r - kHalfRows) * kOB;
@@ -303,13 +331,12 @@ gemm_kernel(const bf16 *__restrict__ a, int64_t lda, const bf16 *__restrict__ w,
       }
     }
     __syncthreads();
-    static_assert((kTM * kChunks) % (64 * kWaves) == 0, "whole store rounds");
 #pragma unroll
-    for (int i = 0; i < kTM * kChunks / (64 * kWaves); ++i) {
+    for (int i = 0; i < (kTM * kChunks + 64 * kWaves - 1) / (64 * kWaves); ++i) {
       const int idx = i * 64 * kWaves + threadIdx.x;
       const int rl = idx / kChunks, c = idx % kChunks;
       const int row = m0 + rl, col = n0 + c * 8;
-      if (row >= M || col >= N) continue;
+      if (rl >= kTM || row >= M || col >= N) continue;
       const u32x4 word = *reinterpret_cast<const u32x4 *>(staged(rl) + ((c ^ (rl & kSw)) << 4));
       *reinterpret_cast<u32x4 *>(out + (int64_t)row * ldo + col) = word;
       if constexpr (kRope) {
@@ -371,9 +398,9 @@ gemm_kernel(const bf16 *__restrict__ a, int64_t lda, const bf16 *__restrict__ w,
   }
 }
 
-template <int TM, int TN, int WM, int WN>
+template <int TM, int TN, int WM, int WN, int Stages, bool kRope>
 int launch_gemm_cfg(const bf16 *a, int64_t lda, const bf16 *w, int64_t ldw, bf16 *out, int64_t ldo,
-                    int64_t M, int64_t N, int64_t K, hipStream_t stream, const RopeKV *rope = nullptr) {
+                    int64_t M, int64_t N, int64_t K, hipStream_t stream, const RopeKV &rope) {
   const int64_t tiles_m = cdiv(M, TM), tiles_n = cdiv(N, TN);
   // With fewer row tiles than XCDs the remap would put every tile on a few
   // XCDs; the plain order spreads the column tiles instead.
@@ -382,40 +409,63 @@ int launch_gemm_cfg(const bf16 *a, int64_t lda, const bf16 *w, int64_t ldw, bf16
   const bool vec = N % 4 == 0 && ldo % 4 == 0 && ((uintptr_t)out & 7) == 0;
   const bool vec16 = N % 8 == 0 && ldo % 8 == 0 && ((uintptr_t)out & 15) == 0;
   const dim3 grid((unsigned)blocks);
-  auto go = [&](auto store_c, auto rope_c) {
-    gemm_kernel<TM, TN, WM, WN, decltype(store_c)::value, decltype(rope_c)::value>
+  auto go = [&](auto store_c) {
+    gemm_kernel<TM, TN, WM, WN, Stages, decltype(store_c)::value, kRope>
         <<<grid, 64 * WM * WN, 0, stream>>>(a, lda, w, ldw, out, ldo, (int)M, (int)N, (int)K,
-                                            (int)tiles_m, (int)tiles_n, (int)remap,
-                                            rope ? *rope : RopeKV{});
+                                            (int)tiles_m, (int)tiles_n, (int)remap, rope);
   };
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;
   using S2 = std::integral_constant<int, 2>;
-  if (rope) {
+  if constexpr (kRope) {
     if (!vec) return LM_EINVAL;
-    if (vec16 && rope->table_len > 0) go(S2{}, std::true_type{});
-    else go(S1{}, std::true_type{});
+    if (vec16 && rope.table_len > 0) go(S2{});
+    else go(S1{});
   } else if (vec16) {
-    go(S2{}, std::false_type{});
+    go(S2{});
   } else if (vec) {
-    go(S1{}, std::false_type{});
+    go(S1{});
   } else {
-    go(S0{}, std::false_type{});
+    go(S0{});
   }
   LM_CHECK_LAUNCH();
   return LM_OK;
 }
 
-// Prefill-sized row counts take 256 x 256 tiles on 16 waves of 64 x 64 (four
-// waves per SIMD). On one box at the cfg 4 QKV shape (46,990 x 1536 x 2560):
-// 443 us against 509 us for 8 waves of 64 x 128 (two per SIMD), 539-587 us
-// for 128 x 256 / 256 x 128 on 16 waves; at the o_proj shape 280 against
-// 326 us. Fewer rows keep 128 x 128 tiles, whose grid spreads over more CUs.
-int launch_gemm_rope(const bf16 *a, int64_t lda, const bf16 *w, int64_t ldw, bf16 *out, int64_t ldo,
-                     int64_t M, int64_t N, int64_t K, hipStream_t stream, const RopeKV *rope) {
-  if (M >= 2048)
-    return launch_gemm_cfg<256, 256, 4, 4>(a, lda, w, ldw, out, ldo, M, N, K, stream, rope);
-  return launch_gemm_cfg<128, 128, 2, 2>(a, lda, w, ldw, out, ldo, M, N, K, stream, rope);
+// The tile is the smallest whose grid the chip holds at once (its workgroups
+// per CU times 256), so that a launch is one round of workgroups, each with
+// little to do, until the operand re-reads of small tiles cost more than idle
+// CUs: below that a launch takes its K loop's latency whatever its size. Up
+// to 16 rows (the LM head of a few prompts) the weights are all the traffic
+// and the tile's rows are mostly padding. Every tile sums K in the same
+// order, so the choice changes no bits. Measured alone on one box, us
+// (before: 128 x 128 tiles on 4 waves below 2048 rows, 256 x 256 above):
+//   rows   N x K         before  now          rows   N x K         before  now
+//   3      49155 x 1536  31.7    27.0         1500   2560 x 1536   24.9    19.4
+//   129    2560 x 1536   17.4     7.9         2047   2560 x 1536   25.2    21.3
+//   300    1536 x 1536   17.2     8.0         4000   2560 x 1536   37.7    33.9
+//   675    2560 x 1536   18.2    11.9         4000   1536 x 1536   25.5*   22.6
+//   1000   1024 x 1024   13.1     6.9         200    49155 x 1536  75.6    57.9
+// (* 128 x 128.) 256 x 256 tiles sit on 16 waves of 64 x 64, four per SIMD:
+// 46,990 x 1536 -> 2560 347 us against 371 us for 192 x 128 and 427 us for
+// 128 x 128 on 4 waves.
+template <bool kRope>
+int launch_gemm_tiled(const bf16 *a, int64_t lda, const bf16 *w, int64_t ldw, bf16 *out, int64_t ldo,
+                      int64_t M, int64_t N, int64_t K, hipStream_t stream, const RopeKV &rope) {
+  auto tiles = [&](int64_t tm, int64_t tn) { return cdiv(M, tm) * cdiv(N, tn); };
+  auto pick = [&]() {
+    if constexpr (!kRope) {
+      if (M <= 16) return launch_gemm_cfg<16, 64, 1, 2, 4, false>;
+    }
+    // (a rope wave holds one head: 64 columns)
+    if (tiles(64, 64) <= 256) return launch_gemm_cfg<64, 64, kRope ? 4 : 2, kRope ? 1 : 2, 3, kRope>;
+    if (tiles(128, 64) <= 256) return launch_gemm_cfg<128, 64, 4, 1, 3, kRope>;
+    if (tiles(64, 128) <= 512) return launch_gemm_cfg<64, 128, 2, 2, 3, kRope>;
+    if (tiles(128, 128) <= 512) return launch_gemm_cfg<128, 128, 4, 2, 2, kRope>;
+    if (tiles(192, 128) <= 512) return launch_gemm_cfg<192, 128, 4, 2, 2, kRope>;
+    return launch_gemm_cfg<256, 256, 4, 4, 2, kRope>;
+  };
+  return pick()(a, lda, w, ldw, out, ldo, M, N, K, stream, rope);
 }
 
 }  // namespace
@@ -429,7 +479,7 @@ bool gemm_shape_ok(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) {
 
 int launch_gemm(const bf16 *a, int64_t lda, const bf16 *w, int64_t ldw, bf16 *out, int64_t ldo,
                 int64_t M, int64_t N, int64_t K, hipStream_t stream) {
-  return launch_gemm_rope(a, lda, w, ldw, out, ldo, M, N, K, stream, nullptr);
+  return launch_gemm_tiled<false>(a, lda, w, ldw, out, ldo, M, N, K, stream, RopeKV{});
 }
 
 }  // namespace lm
@@ -454,8 +504,8 @@ extern "C" int lm_linear_rope_kv(const void *a, int64_t lda, const void *weight,
   LM_REQUIRE((k_cache == nullptr) == (v_cache == nullptr));
   const RopeKV rope{positions, slots, active, (const bf16 *)cos_sin, table_len, (bf16 *)k_cache,
                     (bf16 *)v_cache, capacity, cache_batch, (int)q_heads, (int)kv_heads};
-  return launch_gemm_rope((const bf16 *)a, lda, (const bf16 *)weight, in_features, (bf16 *)qkv, ldo, rows,
-                          n, in_features, (hipStream_t)stream, &rope);
+  return launch_gemm_tiled<true>((const bf16 *)a, lda, (const bf16 *)weight, in_features, (bf16 *)qkv, ldo,
+                                 rows, n, in_features, (hipStream_t)stream, rope);
 }
 
 extern "C" int lm_linear(const void *a, int64_t lda, const void *weight, int64_t ldw, int64_t rows,
