@@ -13,19 +13,16 @@
 // the whole buffer.
 //
 // Workgroup = (output column tile, route block). It computes a kTM x kTN
-// fp32 tile (256 x 256 on 8 waves, or 128 x 128 on 4, see LargeTile /
-// SmallTile): for gate_up the B tile is kTN/2 gate rows and the kTN/2 up rows
+// fp32 tile (see the tiles below): for gate_up the B tile is kTN/2 gate rows and the kTN/2 up rows
 // of the same j, so silu(g)*u is formed in registers. The waves sit in
 // kWM x kWN, each (kTM/kWM) x (kTN/kWN) as 16 x 16 tiles of
 // v_mfma_f32_16x16x32_bf16.
 //
-// K runs in steps of 64. With two LDS stages (the large tile) the next
-// step's A rows (gathered through the route list: each lane's copy has its
-// own address) and B rows are copied from global memory straight into the
-// other stage (global_load_lds_dwordx4, lds_copy16) while the MFMAs run on
-// the current one; with one stage (the small tile) they are loaded into
-// registers meanwhile and stored to LDS after a barrier. An LDS row is 64
-// bf16 = 8 chunks of 16 bytes; chunk c of tile row r sits at position
+// K runs in steps of 64. The next step's A rows (gathered through the route
+// list: each lane's copy has its own address) and B rows are copied from
+// global memory straight into another of the LDS stages
+// (global_load_lds_dwordx4, lds_copy16) while the MFMAs run on the current
+// one. An LDS row is 64 bf16 = 8 chunks of 16 bytes; chunk c of tile row r sits at position
 // c ^ (r & 7), so the 16 rows read by one MFMA fragment load spread over the
 // banks, and each wave instruction fills 1 KB contiguously.
 //
@@ -43,53 +40,83 @@ constexpr int kBK = 64;   // K per stage
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, each with its own L2
 constexpr int kRowBytes = kBK * 2;  // 128
 
-// Two workgroup tiles, chosen per call by the routes per expert:
-// - Large: 256 route rows x 256 B rows on 8 waves of 64 x 128 (4 x 2), two
-//   LDS stages (128 KB, one workgroup per CU): a wave's fragments feed 32
-//   MFMAs per 32-wide k step, half the LDS reads per MFMA of a 64 x 64 wave
-//   tile. At cfg 4's 46,990 tokens (uniform routes, one box, register
-//   staging): gate/up 1230 against 1561 us, down 912 against 1063 us for the
-//   small tile; 16 waves of 64 x 64 1339 / 936 us, 128 x 256 on 8 waves
-//   1412 / 1071 us. With the direct copies the MoE takes 2.13 against 2.34
-//   ms; 16 waves of 64 x 64 (LM_EXPERT_LARGE_WN=4) are within 1% of 8.
-// - Small: 128 x 128 on 4 waves of 64 x 64, one LDS stage (33 KB, several
-//   workgroups per CU), for fewer than 1024 routes per expert, where a
-//   256-route block would be mostly padding.
-// (Earlier measurements of this kernel at 65k tokens: 128 x 128 with two
-// stages 3.83 against 3.34 ms for the MoE; 256 x 256 on 4 waves with the
-// accumulators in AGPRs 4.16 ms.)
 template <int TM, int TN, int WMv, int WNv, int StagesV>
 struct TileCfg {
   static constexpr int M = TM, N = TN, WM = WMv, WN = WNv, Stages = StagesV;
 };
-#ifndef LM_EXPERT_LARGE_WN
-#define LM_EXPERT_LARGE_WN 2
-#endif
-using LargeTile = TileCfg<256, 256, 4, LM_EXPERT_LARGE_WN, 2>;
-using SmallTile = TileCfg<128, 128, 2, 2, 1>;
-constexpr int64_t kLargeTileRoutesPerExpert = 1024;
+// Workgroup tiles, chosen per call by r, the mean routes per expert (what the
+// host knows). An expert's last block is partly padding, so the tile's height
+// follows r; every tile sums K in the same order, so the choice changes no
+// bits. Measured alone on one box, us per launch, gate_up / down, at 40
+// experts, hidden 1536, uniform routes ("before": one 128 x 128 tile on 4
+// waves with register staging below r = 1024, the grid's blocks dealt to the
+// XCDs, 256 x 256 above):
+//      r    before        64 rows     192 rows    256 x 256
+//     30    37.7 / 23.5   29.0 / 12.7  37.9 / 14.6   39.0 / 19.0
+//    140    58.1 / 30.2   44.3 / 23.2  43.5 / 18.2   43.7 / 20.8
+//    400    84.1 / 46.8   80.6 / 44.4  70.3 / 44.9   83.0 / 40.7
+//   1200   161.4 / 96.0      -        156.1 / 99.9  169.3 / 96.1
+// - Low: the weights are read once per block and bound the launch; gate_up
+//   (24 K steps) takes three stages so that two steps' loads are in flight,
+//   down (8 steps) two.
+// - Mid: gate_up 192 x 128 on 8 waves of 48 x 64, 80 KB: two workgroups share
+//   a CU and one computes while the other waits at its barrier. down (one
+//   third of the K steps, three times the output) 192 x 256, whose activation
+//   rows are read by half as many column tiles.
+// - High: 256 x 256 on 8 waves, a wave's 12 fragment reads feed 32 MFMAs:
+//   down 128 x 64 waves (665 -> 655 us at r = 9400, skewed routes, against
+//   64 x 128), gate_up 64 x 128 (978 against 985 us).
+using GateLow = TileCfg<64, 256, 2, 4, 3>;
+using GateMid = TileCfg<192, 128, 4, 2, 2>;
+using DownLow = TileCfg<64, 128, 2, 2, 2>;
+using DownMid = TileCfg<192, 256, 4, 2, 2>;
+using DownMidNarrow = TileCfg<192, 128, 4, 2, 2>;  // hidden not a multiple of 256
+using GateHigh = TileCfg<256, 256, 4, 2, 2>;
+using DownHigh = TileCfg<256, 256, 2, 4, 2>;
+constexpr int64_t kLowBelow = 96, kGateHighFrom = 2048, kDownHighFrom = 1024;
 
-// Block b of the per-expert blocks of bm routes (offsets: exclusive prefix
-// of per-expert counts, as lm_moe_align writes it), found by each wave with
-// one vector load per 64 experts: lane l takes expert e0 + l's block count,
-// an inclusive prefix sum over the lanes gives each expert's first block, and
-// the expert holding b is the one lane whose block range contains it. (A
-// scalar walk over the experts waits on one load per expert.)
+// The route block of workgroup `lin` (blocks of at most bm routes of one
+// expert, from the offsets lm_moe_align writes: exclusive prefix of the
+// per-expert counts), numbered so that each XCD takes an eighth of the blocks
+// there are: workgroups are dealt to the 8 XCDs round-robin in launch order,
+// so workgroup lin is number lin / 8 of XCD lin % 8, and takes block (that
+// XCD's first) + number / cols. The grid is sized for the most blocks the
+// routes can make; dealing out the grid's blocks instead of the existing ones
+// would leave the last XCDs the empty ones (gate/up at 300 tokens over 40
+// experts: 55 of 80 blocks exist).
+// Lane l takes expert e0 + l's block count; an inclusive prefix sum over the
+// lanes gives each expert's first block, and the expert holding the block is
+// the one lane whose range contains it. (A scalar walk over the experts waits
+// on one load per expert.)
 __device__ __forceinline__ bool block_of(const int32_t *__restrict__ offsets, int experts, int bm,
-                                         int b, int &e_out, int &r0, int &r1) {
+                                         int lin, int cols, int &e_out, int &r0, int &r1) {
   const int lane = threadIdx.x % kWave;
-  int before = 0;  // blocks of the experts below e0
-  for (int e0 = 0; e0 < experts; e0 += kWave) {
+  auto counts = [&](int e0, int &o0, int &o1, int &incl) {  // returns the lane's own count
     const int e = e0 + lane;
-    const int o0 = e < experts ? offsets[e] : 0;
-    const int o1 = e < experts ? offsets[e + 1] : 0;
+    o0 = e < experts ? offsets[e] : 0;
+    o1 = e < experts ? offsets[e + 1] : 0;
     const int nb = (o1 - o0 + bm - 1) / bm;
-    int incl = nb;
+    incl = nb;
 #pragma unroll
     for (int d = 1; d < kWave; d *= 2) {
       const int up = __shfl_up(incl, d, kWave);
       if (lane >= d) incl += up;
     }
+    return nb;
+  };
+  int o0, o1, incl;
+  int nb = counts(0, o0, o1, incl);
+  int total = __shfl(incl, kWave - 1, kWave);
+  for (int e0 = kWave; e0 < experts; e0 += kWave) {
+    int p0, p1, more;
+    counts(e0, p0, p1, more);
+    total += __shfl(more, kWave - 1, kWave);
+  }
+  const int per_xcd = (total + kXcds - 1) / kXcds, j = lin / kXcds / cols;
+  const int b = (lin % kXcds) * per_xcd + j;
+  if (j >= per_xcd || b >= total) return false;
+  int before = 0;  // blocks of the experts below e0
+  for (int e0 = 0;;) {
     const int first = before + incl - nb;
     const uint64_t hit = __ballot(b >= first && b < first + nb);
     if (hit) {
@@ -100,8 +127,10 @@ __device__ __forceinline__ bool block_of(const int32_t *__restrict__ offsets, in
       return true;
     }
     before += __shfl(incl, kWave - 1, kWave);
+    e0 += kWave;
+    if (e0 >= experts) return false;
+    nb = counts(e0, o0, o1, incl);
   }
-  return false;
 }
 
 // Byte offset in an operand tile of (row, 16-byte chunk).
@@ -127,27 +156,23 @@ expert_gemm_kernel(const bf16 *__restrict__ a_src, const bf16 *__restrict__ w,
   constexpr int kWaves = kWM * kWN, kThreadsT = 64 * kWaves;
   constexpr int kWaveRows = kTM / kWM, kWaveCols = kTN / kWN;
   constexpr int kRB = kWaveRows / 16, kCB = kWaveCols / 16;  // 16-row / 16-column blocks per wave
-  constexpr int kLA = kTM / (8 * kWaves), kLB = kTN / (8 * kWaves);  // 16-byte loads per lane
-  static_assert(kLA * 8 * kWaves == kTM && kLB * 8 * kWaves == kTN, "tile rows per load round");
+  constexpr int kLA = kTM / (8 * kWaves), kLB = kTN / (8 * kWaves);  // 16-byte copies per lane
+  static_assert(kLA * 8 * kWaves == kTM && kLB * 8 * kWaves == kTN, "tile rows per copy round");
   static_assert(!kGateUp || kCB % 2 == 0, "gate/up waves hold gate and up blocks in pairs");
   constexpr int kABytes = kTM * kRowBytes, kStageBytes = (kTM + kTN) * kRowBytes;
-  // kStages == 2: two LDS stages filled by direct copies; kStages == 1: one,
-  // filled from registers.
-  __shared__ __align__(16) char smem[kStageBytes];
+  // two stages are two arrays, three one array
+  __shared__ __align__(16) char smem[kStages == 2 ? kStageBytes : kStages * kStageBytes];
   __shared__ __align__(16) char smem1[kStages == 2 ? kStageBytes : 16];
   __shared__ int route_of[kTM];
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  // Workgroups are dealt to the 8 XCDs round-robin in launch order. Remap so
-  // that each XCD takes a contiguous range of route blocks with all their
-  // column tiles: a block's gathered A rows are then fetched into one L2, and
-  // an expert's weight rows mostly into one or two.
+  // Each XCD takes a contiguous range of route blocks with all their column
+  // tiles (block_of): a block's gathered A rows are then fetched into one L2,
+  // and an expert's weight rows mostly into one or two.
   const int cols = gridDim.x;
   const int lin = blockIdx.y * cols + blockIdx.x;
-  const int j = lin / kXcds;  // gridDim.y is a multiple of kXcds
-  const int tile_y = (lin % kXcds) * (gridDim.y / kXcds) + j / cols;
-  const int tile_x = j % cols;
+  const int tile_x = lin / kXcds % cols;  // gridDim.y is a multiple of kXcds
   int e, r0, r1;
-  if (!block_of(offsets, experts, kTM, tile_y, e, r0, r1)) return;
+  if (!block_of(offsets, experts, kTM, lin, cols, e, r0, r1)) return;
   const int n = r1 - r0;
   const int c0 = tile_x * (kGateUp ? kTN / 2 : kTN);  // first output column
   // The route list in LDS serves the A row offsets of gate_up and of down on
@@ -188,27 +213,8 @@ expert_gemm_kernel(const bf16 *__restrict__ a_src, const bf16 *__restrict__ w,
   }
   // element advance of one kBK step of B (two 32-wide k-steps when packed)
   constexpr int kBStep = kPacked ? (int)(kBK / 32 * wstep<true>()) : kBK;
-  // One stage: step k+1 is loaded into registers while step k is computed
-  // from LDS, then stored to LDS after a barrier.
-  u32x4 ra[kLA], rbv[kLB];
-  auto load = [&](int kt) {
-    const int k0 = kt * kBK;
-#pragma unroll
-    for (int i = 0; i < kLA; ++i) ra[i] = *reinterpret_cast<const u32x4 *>(a_src + oa[i] + k0);
-#pragma unroll
-    for (int i = 0; i < kLB; ++i) rbv[i] = *reinterpret_cast<const u32x4 *>(w + ob[i] + kt * kBStep);
-  };
-  auto store = [&]() {
-    char *base = smem + lane * 16;
-#pragma unroll
-    for (int i = 0; i < kLA; ++i) *reinterpret_cast<u32x4 *>(base + (wave * kLA + i) * 1024) = ra[i];
-#pragma unroll
-    for (int i = 0; i < kLB; ++i)
-      *reinterpret_cast<u32x4 *>(base + kABytes + (wave * kLB + i) * 1024) = rbv[i];
-  };
-  // Two stages: step k+1 is copied from global memory straight into the
-  // other stage while step k is computed (byte offsets: the element offsets
-  // are below 2^31).
+  // A step's rows from global memory straight into an LDS stage (byte
+  // offsets: the element offsets are below 2^31).
   const uint32_t uw = __builtin_amdgcn_readfirstlane(wave);
   auto issue_a = [&](int kt, const char *stage) {
     const bf16 *ak = a_src + kt * kBK;
@@ -308,19 +314,30 @@ expert_gemm_kernel(const bf16 *__restrict__ a_src, const bf16 *__restrict__ w,
       }
     }
   } else {
-    load(0);
+    // A ring: the copies of kStages - 1 steps are in flight; a step waits for
+    // its own only (they complete in issue order), and one barrier tells that
+    // every wave's copies have landed and that every wave has left the step
+    // whose slot the next copy goes into.
+    static_assert(kStages == 3, "the wait below leaves one later step in flight");
+    constexpr int kL = kLA + kLB;  // copies of one step per wave
+    auto issue = [&](int kt, const char *stage) {
+      issue_a(kt, stage);
+      issue_b(kt, stage);
+    };
+#pragma unroll
+    for (int s = 0; s < kStages - 1; ++s)
+      if (s < nk) issue(s, smem + s * kStageBytes);
     if constexpr (kRouteList && !kListFirst) fill_routes();
-    store();
-    __syncthreads();
-    for (int kt = 0; kt + 1 < nk; ++kt) {
-      load(kt + 1);
-      __builtin_amdgcn_sched_barrier(0);  // the loads go out before the MFMAs
-      compute(smem);
-      __syncthreads();  // every wave is done with the buffer
-      store();
+    int cur = 0, nxt = (kStages - 1) * kStageBytes;
+    for (int kt = 0; kt < nk; ++kt) {
+      if (kt + 1 < nk) vm_wait<kL>(); else vm_wait<0>();
       __syncthreads();
+      if (kt + kStages - 1 < nk) issue(kt + kStages - 1, smem + nxt);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(smem + cur);
+      cur = cur == (kStages - 1) * kStageBytes ? 0 : cur + kStageBytes;
+      nxt = nxt == (kStages - 1) * kStageBytes ? 0 : nxt + kStageBytes;
     }
-    compute(smem);
   }
 
   // Transposed C fragment: lane holds output row lane%16 of each 16-row block
@@ -334,8 +351,8 @@ expert_gemm_kernel(const bf16 *__restrict__ a_src, const bf16 *__restrict__ w,
   // the 16 rows of one fragment store fall on different bank groups.
   constexpr int kOutCols = kGateUp ? kTN / 2 : kTN, kOB = kOutCols * 2;  // output row bytes
   constexpr int kChunks = kOB / 16, kSw = (kChunks < 16 ? kChunks : 16) - 1;
-  constexpr int kHalfRows = kStageBytes / kOB;  // rows held by the first stage
-  static_assert(kTM * kOB <= (kStages == 2 ? 2 : 1) * kStageBytes, "output tile fits the LDS stages");
+  constexpr int kHalfRows = (kStages == 2 ? 1 : kStages) * kStageBytes / kOB;  // rows held by smem
+  static_assert(kTM * kOB <= kStages * kStageBytes, "output tile fits the LDS stages");
   auto staged = [&](int row) -> char * {
     if constexpr (kTM <= kHalfRows) return smem + row * kOB;
     else return row < kHalfRows ? smem + row * kOB : smem1 + (row - kHalfRows) * kOB;
@@ -366,9 +383,8 @@ expert_gemm_kernel(const bf16 *__restrict__ a_src, const bf16 *__restrict__ w,
     }
   }
   __syncthreads();
-  static_assert((kTM * kChunks) % kThreadsT == 0, "whole store rounds");
 #pragma unroll
-  for (int i = 0; i < kTM * kChunks / kThreadsT; ++i) {
+  for (int i = 0; i < (kTM * kChunks + kThreadsT - 1) / kThreadsT; ++i) {
     const int idx = i * kThreadsT + threadIdx.x;
     const int row = idx / kChunks, c = idx % kChunks;
     if (row >= n) continue;
@@ -388,7 +404,7 @@ bool expert_gemm_ok(int64_t routes, int64_t hidden, int64_t inter, int64_t exper
   // 32-bit element offsets: the gathered rows and the weights stay below 2^31.
   const int64_t rows = std::max(routes, experts * std::max(2 * inter, hidden));
   return routes >= kExpertGemmMinRoutes && hidden % kBK == 0 && inter % kBK == 0 &&
-         (2 * inter) % SmallTile::N == 0 && hidden % SmallTile::N == 0 &&
+         (2 * inter) % GateLow::N == 0 && hidden % DownLow::N == 0 &&
          rows * std::max(hidden, inter) < ((int64_t)1 << 31);
 }
 
@@ -424,18 +440,15 @@ int launch_tile(bool gate_up, const bf16 *a, const bf16 *w, const int32_t *offse
   return LM_OK;
 }
 
-bool large_tile(int64_t routes, int64_t hidden, int64_t inter, int64_t experts) {
-  return routes >= kLargeTileRoutesPerExpert * experts && (2 * inter) % LargeTile::N == 0 &&
-         hidden % LargeTile::N == 0;
-}
-
 }  // namespace
 
 int launch_expert_gemm_gate_up(const bf16 *x, const bf16 *w13, const int32_t *offsets,
                                const int32_t *sorted, int64_t routes, int64_t topk, int64_t hidden,
                                int64_t inter, int64_t experts, bf16 *act, bool packed,
                                bool sorted_act, hipStream_t stream) {
-  auto launch = large_tile(routes, hidden, inter, experts) ? launch_tile<LargeTile> : launch_tile<SmallTile>;
+  auto launch = routes < kLowBelow * experts        ? launch_tile<GateLow>
+                : routes < kGateHighFrom * experts ? launch_tile<GateMid>
+                                                   : launch_tile<GateHigh>;
   return launch(true, x, w13, offsets, sorted, routes, topk, hidden, inter, inter, experts, act,
                 packed, sorted_act, stream);
 }
@@ -444,7 +457,11 @@ int launch_expert_gemm_down(const bf16 *act, const bf16 *w2, const int32_t *offs
                             const int32_t *sorted, int64_t routes, int64_t hidden, int64_t inter,
                             int64_t experts, bf16 *y, bool packed, bool sorted_act,
                             hipStream_t stream) {
-  auto launch = large_tile(routes, hidden, inter, experts) ? launch_tile<LargeTile> : launch_tile<SmallTile>;
+  const bool wide = hidden % DownMid::N == 0;
+  auto launch = routes < kLowBelow * experts ? launch_tile<DownLow>
+                : !wide                      ? launch_tile<DownMidNarrow>
+                : routes < kDownHighFrom * experts ? launch_tile<DownMid>
+                                                   : launch_tile<DownHigh>;
   return launch(false, act, w2, offsets, sorted, routes, 1, inter, hidden, inter, experts, y, packed,
                 sorted_act, stream);
 }
