@@ -6,6 +6,8 @@
 // Weights follow vLLM fused_topk / HF GraniteMoeTopKRouter: softmax over the
 // k selected logits (renormalize) or over all E logits.
 // References: litemoe/model.py:110-118, ops.py:7-12, ops.py:163-173.
+#include <algorithm>
+
 #include "internal.h"
 
 namespace lm {
@@ -162,7 +164,7 @@ __device__ void select_topk_lanes(const float *logit, float *scratch, int t, int
     }
   } else {
     if (t < experts) terms[t] = ex;
-#pragma unroll
+#pragma unroll 4
     for (int e4 = 0; e4 < kWave / 4; ++e4) {
       const float4 t4 = *reinterpret_cast<const float4 *>(terms + 4 * e4);
       const float tv[4] = {t4.x, t4.y, t4.z, t4.w};
@@ -568,30 +570,34 @@ template <int NVL, bool kAdd>
 __device__ __forceinline__ void batch_norm_row(bf16 *__restrict__ x, float alpha,
                                                const u32x4 (&gv)[NVL], float eps,
                                                bf16 *__restrict__ z, int64_t row,
-                                               const u32x4 (&xv)[NVL], const u32x4 (&av)[NVL]) {
+                                               const u32x4 (&xv)[NVL], const u32x4 (&av)[NVL],
+                                               u32x4 *staged = nullptr) {
   constexpr int kJ = NVL < kRouterWaves ? NVL : kRouterWaves;
   const int lane = threadIdx.x % kWave;
   u32x4 *xr = reinterpret_cast<u32x4 *>(x) + row * NVL * kWave;
   u32x4 *zr = reinterpret_cast<u32x4 *>(z) + row * NVL * kWave;
-  float xn[NVL][8];
+  u32x4 xo[NVL];  // the new x: bf16 values, so half the registers lose nothing
   float ss[kJ];
 #pragma unroll
   for (int j = 0; j < kJ; ++j) ss[j] = 0.f;
 #pragma unroll
   for (int i = 0; i < NVL; ++i) {
-    unpack8(xv[i], xn[i]);
+    float xn[8];
+    unpack8(xv[i], xn);
+    xo[i] = xv[i];
     if constexpr (kAdd) {
       float g[8];
       unpack8(av[i], g);
-      u32x4 o;
 #pragma unroll
-      for (int c = 0; c < 8; ++c) xn[i][c] = round_bf16(xn[i][c] + alpha * g[c]);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) o[c] = pack_bf16(xn[i][2 * c], xn[i][2 * c + 1]);
-      xr[lane + i * kWave] = o;
+      for (int c = 0; c < 4; ++c) {
+        xo[i][c] = pack_bf16(xn[2 * c] + alpha * g[2 * c], xn[2 * c + 1] + alpha * g[2 * c + 1]);
+        xn[2 * c] = lo_f32(xo[i][c]);
+        xn[2 * c + 1] = hi_f32(xo[i][c]);
+      }
+      xr[lane + i * kWave] = xo[i];
     }
 #pragma unroll
-    for (int c = 0; c < 8; ++c) ss[i % kRouterWaves] += xn[i][c] * xn[i][c];
+    for (int c = 0; c < 8; ++c) ss[i % kRouterWaves] += xn[c] * xn[c];
   }
   float total = 0.f;
 #pragma unroll
@@ -599,14 +605,16 @@ __device__ __forceinline__ void batch_norm_row(bf16 *__restrict__ x, float alpha
   const float scale = 1.0f / sqrtf(total / (float)(NVL * 512) + eps);
 #pragma unroll
   for (int i = 0; i < NVL; ++i) {
-    float g[8];
+    float xn[8], g[8];
+    unpack8(xo[i], xn);
     unpack8(gv[i], g);
     u32x4 o;
 #pragma unroll
     for (int c = 0; c < 4; ++c)
-      o[c] = pack_bf16(round_bf16(xn[i][2 * c] * scale) * g[2 * c],
-                       round_bf16(xn[i][2 * c + 1] * scale) * g[2 * c + 1]);
+      o[c] = pack_bf16(round_bf16_nc(xn[2 * c] * scale) * g[2 * c],
+                       round_bf16_nc(xn[2 * c + 1] * scale) * g[2 * c + 1]);
     zr[lane + i * kWave] = o;
+    if (staged) staged[lane + i * kWave] = o;
   }
 }
 
@@ -698,7 +706,157 @@ batched_router_kernel(bf16 *__restrict__ x, const bf16 *__restrict__ a, float al
                       tw + (row0 + r) * topk, tid + (row0 + r) * topk);
 }
 
-// Routes the first tokens - tokens % kBatchRows tokens with
+// The same three phases as a persistent kernel: 256 workgroups of sixteen
+// waves, each over every 256th block of 16 tokens, a token per wave. Wave w
+// holds the K quarter w % 4 of gate tile w / 4 as MFMA B operands for the
+// whole launch, so no block reads the gate weights again;
+// a block's z rows reach the matrix cores through LDS (rows padded by 16
+// bytes: a fragment's 16 rows fall on 16 bank groups) instead of being read
+// back from L2; and the next block's row is in flight from the moment the norm
+// has taken this block's, so HBM streams under the logits and the selection
+// instead of alternating with them. The last tokens % 16 are routed beside the
+// blocks in the per-token kernels' order, so there is no tail launch; the
+// blocks' x, z and logits are bitwise batched_router_kernel's. The stream bounds it: 577 MB at 46,990
+// tokens of hidden 1536, 40 experts, in 121 us (4.8 TB/s; a large copy
+// reaches 4.9) against 162 us for batched_router_kernel and its tail launch;
+// 2000 tokens 35 -> 13 us; hidden 1024, 32 experts, 46,990 tokens 107 -> 79
+// us. Eight waves of two tokens, each holding its quarter of all gate tiles
+// (two waves per SIMD to hide latency with): 166 us. From hidden 2048 the
+// weights no longer fit beside the rows, and batched_router_kernel stays.
+constexpr int kPersistWaves = 16, kPersistThreads = kPersistWaves * kWave, kPersistRows = 16;
+constexpr int64_t kPersistGrid = 256;
+
+template <int NVL, int NT, bool kNorm, bool kAdd>
+__global__ void __launch_bounds__(kPersistThreads, 1)
+persistent_router_kernel(bf16 *__restrict__ x, const bf16 *__restrict__ a, float alpha,
+                         const bf16 *__restrict__ nw, float eps, bf16 *__restrict__ z,
+                         const bf16 *__restrict__ wr, int64_t tokens, int experts, int topk,
+                         int renormalize, bf16 *__restrict__ logits_out, float *__restrict__ tw,
+                         int32_t *__restrict__ tid) {
+  constexpr int kNvec = NVL * kWave, kWaveSteps = NVL * 4;  // a K quarter's 32-wide k-steps
+  constexpr int kPitch = kNvec + 1;                         // 16-byte words of a staged row
+  static_assert(kBatchWaves * NT <= kPersistWaves, "a wave per K quarter and gate tile");
+  __shared__ u32x4 zs[kPersistRows * kPitch];
+  __shared__ u32x4 gs[kNorm ? kNvec : 1];  // the norm weight
+  // k-steps whose gate fragments a wave holds in registers; the rest in LDS
+  // (twelve held at hidden 1536 spill four, and their reload from scratch
+  // waits behind the row in flight: 141 us at 46,990 tokens)
+  constexpr int kHeld = kWaveSteps < 8 ? kWaveSteps : 8;
+  __shared__ u32x4 bl[kPersistWaves][kWaveSteps > kHeld ? kWaveSteps - kHeld : 1][kWave];
+  __shared__ __align__(16) float part[kBatchWaves][NT][4][kWave];
+  __shared__ __align__(16) float logit[kPersistWaves][NT * 16];
+  __shared__ __align__(16) float scratch[kPersistWaves][2 * kWave];
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int tr = lane % 16, kg = lane / 16;
+  const int kq = wave % kBatchWaves, nt = wave / kBatchWaves;  // nt >= NT: no logits
+  const int64_t blocks = tokens / kPersistRows;  // whole blocks
+  int64_t row = (int64_t)blockIdx.x * kPersistRows + wave;
+  const int64_t stride = (int64_t)gridDim.x * kPersistRows;
+  u32x4 xv[NVL], av[NVL];
+  batch_load_row<NVL, kAdd>(x, a, min(row, tokens - 1), xv, av);
+  if constexpr (kNorm) {  // published by the barrier before the first block
+    if (threadIdx.x < kNvec) gs[threadIdx.x] = reinterpret_cast<const u32x4 *>(nw)[threadIdx.x];
+    __syncthreads();
+  }
+  const int k0 = kq * kWaveSteps * 4 + kg;  // 16-byte word of the quarter's first k-step
+  u32x4 bw[kHeld];
+  const u32x4 *bp = reinterpret_cast<const u32x4 *>(wr) + (int64_t)min(16 * nt + tr, experts - 1) * kNvec + k0;
+#pragma unroll
+  for (int t = 0; t < kHeld; ++t) bw[t] = bp[4 * t];
+#pragma unroll
+  for (int t = kHeld; t < kWaveSteps; ++t) bl[wave][t - kHeld][lane] = bp[4 * t];  // this wave's own
+  for (int64_t blk = blockIdx.x; blk < blocks; blk += gridDim.x, row += stride) {
+    u32x4 *zrow = zs + wave * kPitch;
+    if constexpr (kNorm) {
+      u32x4 gv[NVL];
+#pragma unroll
+      for (int i = 0; i < NVL; ++i) gv[i] = gs[lane + i * kWave];
+      batch_norm_row<NVL, kAdd>(x, alpha, gv, eps, z, row, xv, av, zrow);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NVL; ++i) zrow[lane + i * kWave] = xv[i];
+    }
+    __builtin_amdgcn_sched_barrier(0);  // into the registers that the norm has left
+    if (blk + gridDim.x < blocks) batch_load_row<NVL, kAdd>(x, a, min(row + stride, tokens - 1), xv, av);
+    __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    if (nt < NT) {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < kWaveSteps; ++t) {
+        acc = mfma16x16x32(zs[tr * kPitch + k0 + 4 * t], t < kHeld ? bw[t % kHeld] : bl[wave][t - kHeld][lane], acc);
+        // at most four fragments read ahead: all at once would spill
+        if (t % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) part[kq][nt][i][lane] = acc[i];
+    }
+    __syncthreads();
+    // Wave w sums and selects row w. C layout: lane l of a tile holds rows
+    // 4*(l/16) + i of column l % 16. The next block's writes of zs come after
+    // every wave's fragment reads (the barrier above), and of part after every
+    // wave's sums (the next block's first barrier).
+    if (lane < NT * 16) {
+      const int n = lane / 16, l = 16 * (wave / 4) + lane % 16;
+      float sum = part[0][n][wave % 4][l];
+#pragma unroll
+      for (int w = 1; w < kBatchWaves; ++w) sum += part[w][n][wave % 4][l];
+      const uint32_t h = f32_to_bf16(sum);
+      logit[wave][lane] = bf16_to_f32(h);
+      if (logits_out && lane < experts) logits_out[row * experts + lane] = (bf16)h;
+    }
+    __builtin_amdgcn_wave_barrier();
+    // opaque copies: hoisted out of the block loop, the selection's many
+    // comparisons with them would spill a hundred scalar registers
+    int n_experts = experts, k = topk;
+    asm volatile("" : "+s"(n_experts), "+s"(k));
+    select_topk_lanes(logit[wave], scratch[wave], lane, n_experts, k, renormalize, tw + row * topk,
+                      tid + row * topk);
+  }
+  // The last tokens % 16: the workgroup whose next block they would be norms a
+  // token per wave and then takes a gate row per wave over all of them, the
+  // logits in the per-token kernels' order (gate_round).
+  const int tail = (int)(tokens % kPersistRows);
+  if (tail == 0 || blockIdx.x != blocks % gridDim.x) return;
+  row = blocks * kPersistRows + wave;
+  if (wave < tail) {
+    batch_load_row<NVL, kAdd>(x, a, row, xv, av);
+    u32x4 *zrow = zs + wave * kPitch;
+    if constexpr (kNorm) {
+      u32x4 gv[NVL];
+#pragma unroll
+      for (int i = 0; i < NVL; ++i) gv[i] = gs[lane + i * kWave];
+      batch_norm_row<NVL, kAdd>(x, alpha, gv, eps, z, row, xv, av, zrow);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NVL; ++i) zrow[lane + i * kWave] = xv[i];
+    }
+  }
+  __syncthreads();  // (also: every wave has selected from logit)
+  for (int e = wave; e < experts; e += kPersistWaves) {
+    u32x4 gw[NVL];
+#pragma unroll
+    for (int i = 0; i < NVL; ++i) gw[i] = reinterpret_cast<const u32x4 *>(wr)[(int64_t)e * kNvec + lane + i * kWave];
+    for (int r = 0; r < tail; ++r) {
+      float acc = 0.f;
+#pragma unroll
+      for (int i = 0; i < NVL; ++i) acc = dot8_bf16_acc(zs[r * kPitch + lane + i * kWave], gw[i], acc);
+      const uint32_t h = f32_to_bf16(wave_sum(acc));
+      if (lane == 0) {
+        logit[r][e] = bf16_to_f32(h);
+        if (logits_out) logits_out[(blocks * kPersistRows + r) * experts + e] = (bf16)h;
+      }
+    }
+  }
+  __syncthreads();
+  if (wave < tail)
+    select_topk_lanes(logit[wave], scratch[wave], lane, experts, topk, renormalize, tw + row * topk,
+                      tid + row * topk);
+}
+
+// Routes every token with persistent_router_kernel, or the first
+// tokens - tokens % kBatchRows tokens with
 // batched_router_kernel when the shape allows it; returns how many it routed
 // (0: none, the per-token kernels route them all).
 template <bool kNorm, bool kAdd>
@@ -708,6 +866,17 @@ int64_t launch_batched_router(int64_t tokens, int64_t hidden, bf16 *x, const bf1
                               float *tw, int32_t *tid, hipStream_t s) {
   const int nv = fast_nv(hidden);
   if (tokens < kBatchRouterMinTokens || !nv || experts > kWave || experts <= 16) return 0;
+#define LM_PERSIST_ROUTER(NVL, NT)                                                               \
+  if (nv == NVL && (experts + 15) / 16 == NT) {                   \
+    const dim3 pgrid((unsigned)std::min(cdiv(tokens, kPersistRows), kPersistGrid));     \
+    persistent_router_kernel<NVL, NT, kNorm, kAdd><<<pgrid, kPersistThreads, 0, s>>>(            \
+        x, a, alpha, nw, eps, z, wr, tokens, experts, topk, renormalize, logits_out, tw, tid);   \
+    return tokens;                                                                               \
+  }
+  LM_PERSIST_ROUTER(1, 2) LM_PERSIST_ROUTER(1, 3) LM_PERSIST_ROUTER(1, 4)
+  LM_PERSIST_ROUTER(2, 2) LM_PERSIST_ROUTER(2, 3) LM_PERSIST_ROUTER(2, 4)
+  LM_PERSIST_ROUTER(3, 2) LM_PERSIST_ROUTER(3, 3) LM_PERSIST_ROUTER(3, 4)
+#undef LM_PERSIST_ROUTER
   const int64_t rows = tokens - tokens % kBatchRows;
   const int nt = (experts + 15) / 16;
   const dim3 grid((unsigned)(rows / kBatchRows));
@@ -820,6 +989,90 @@ align_kernel(const int32_t *__restrict__ ids, int routes, int first, int local,
   }
 }
 
+
+// The same stable argsort for at most kAlignChunkedMinRoutes routes, without
+// a wait per 64 routes: a wave loads all its ids at once (at most
+// kAlignHeld per lane, clamped and masked), finds each route's rank among the
+// wave's equal keys once, in one pass, and keeps key and rank in registers
+// until the bases are known; the bases come from wave prefix sums over 64
+// keys per wave instead of ten barriers of a 1024-thread scan. One load round
+// trip and four barriers: 11.6 -> 7.9 us at 5400 routes, 40 experts, 5.5 -> 4.2
+// at 1032.
+constexpr int kAlignHeld = 8;
+static_assert(kAlignHeld * kWave * kAlignWaves >= kAlignChunkedMinRoutes, "every route is held");
+
+__global__ void __launch_bounds__(kAlignThreads)
+align_held_kernel(const int32_t *__restrict__ ids, int routes, int first, int local,
+                  int32_t *__restrict__ offsets, int32_t *__restrict__ sorted,
+                  int32_t *__restrict__ inverse) {
+  extern __shared__ int cnt[];  // [kAlignWaves][keys]
+  __shared__ int group_total[kAlignWaves];
+  const int keys = local + 1;
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int seg = (int)(cdiv(cdiv(routes, kAlignWaves), kWave) * kWave);
+  const int begin = wave * seg, end = min(routes, begin + seg);
+  int id[kAlignHeld];
+#pragma unroll
+  for (int i = 0; i < kAlignHeld; ++i) id[i] = ids[min(begin + i * kWave + lane, routes - 1)];
+  for (int i = threadIdx.x; i < kAlignWaves * keys; i += kAlignThreads) cnt[i] = 0;
+  __syncthreads();
+  const int nbits = 32 - __clz(local);
+  const uint64_t below = (1ull << lane) - 1ull;
+  int key[kAlignHeld], rank[kAlignHeld];  // rank: among the wave's earlier routes of the key
+#pragma unroll
+  for (int i = 0; i < kAlignHeld; ++i) {
+    key[i] = rank[i] = 0;
+    if (begin + i * kWave >= end) continue;  // wave-uniform
+    const bool valid = begin + i * kWave + lane < end;
+    const int e = id[i] - first;
+    key[i] = valid && e >= 0 && e < local ? e : local;
+    const uint64_t eq = match_key(key[i], valid, nbits);
+    const int at = wave * keys + key[i];
+    const int before = cnt[at], among = __popcll(eq & below);
+    rank[i] = before + among;
+    __builtin_amdgcn_wave_barrier();
+    if (valid && among == 0) cnt[at] = before + __popcll(eq);
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  // Wave g: the keys 64 g .. 64 g + 63 (keys <= 64 * kAlignWaves).
+  const int k = wave * kWave + lane;
+  int c[kAlignWaves], total = 0;
+#pragma unroll
+  for (int w = 0; w < kAlignWaves; ++w) {
+    c[w] = k < keys ? cnt[w * keys + k] : 0;
+    total += c[w];
+  }
+  int incl = total;
+#pragma unroll
+  for (int d = 1; d < kWave; d *= 2) {
+    const int up = __shfl_up(incl, d, kWave);
+    if (lane >= d) incl += up;
+  }
+  if (lane == kWave - 1) group_total[wave] = incl;
+  __syncthreads();
+  int running = incl - total;
+#pragma unroll
+  for (int w = 0; w < kAlignWaves; ++w) running += w < wave ? group_total[w] : 0;
+  if (k < keys) {
+    offsets[k] = running;
+#pragma unroll
+    for (int w = 0; w < kAlignWaves; ++w) {
+      cnt[w * keys + k] = running;
+      running += c[w];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kAlignHeld; ++i) {
+    const int r = begin + i * kWave + lane;
+    if (r < end) {
+      const int pos = cnt[wave * keys + key[i]] + rank[i];
+      sorted[pos] = r;
+      if (inverse) inverse[r] = pos;
+    }
+  }
+}
 
 // The same stable argsort for large route counts, over chunks of 1024 routes
 // (16 waves x 64) in three launches: per-chunk key counts; one workgroup
@@ -1103,6 +1356,9 @@ int launch_align(const int32_t *ids, int64_t routes, int64_t first_expert, int64
     align_scan_kernel<<<1, kScanWaves * kWave, 0, stream>>>(counts, chunks, keys, bases, offsets);
     align_chunk_kernel<true><<<chunks, kChunk, wave_bytes, stream>>>(
         ids, (int)routes, (int)first_expert, (int)local_experts, nullptr, bases, sorted, inverse);
+  } else if (routes > 0 && routes <= kAlignChunkedMinRoutes) {
+    align_held_kernel<<<1, kAlignThreads, wave_bytes, stream>>>(
+        ids, (int)routes, (int)first_expert, (int)local_experts, offsets, sorted, inverse);
   } else {
     align_kernel<<<1, kAlignThreads, wave_bytes + sizeof(int) * 2 * kAlignThreads, stream>>>(
         ids, (int)routes, (int)first_expert, (int)local_experts, offsets, sorted, inverse);

@@ -1,12 +1,13 @@
-"""The tile choices of the prefill GEMMs: every tile of the dense and the
+"""The kernels that prefill calls choose by size: every tile of the dense and the
 expert kernels at sizes that leave remainders in rows, columns and K steps,
-on both sides of the lines between tiles."""
+on both sides of the lines between tiles, the persistent router and the
+route permutation at their limits."""
 import pytest
 import torch
 
 import test_gpu_projections as projections
 from helpers import rel_l2
-from litemoe_amd import experts, linear
+from litemoe_amd import experts, linear, norm, router
 from oracle import ops
 
 pytestmark = pytest.mark.gpu
@@ -69,3 +70,44 @@ def test_expert_gemm_tiles_match_oracle(m, h, i, e, k):
     per_row = (y.cpu().float() - exp.float()).norm(dim=1) / exp.float().norm(dim=1).clamp_min(1e-6)
     assert float(per_row.max()) < 5e-2
     assert torch.equal(experts.moe_routes(d[0], *experts.pack_expert_weights(d[1], d[2]), d[3], packed=True), y)
+
+
+@pytest.mark.parametrize("m,h,e,k,add", [
+    (1024, 1536, 40, 8, True), (1025, 1024, 32, 8, True), (1039, 512, 17, 2, True),
+    (4096, 1024, 33, 4, False), (4096 + 16, 1536, 40, 8, True), (9000 + 15, 1536, 64, 8, True),
+    (2055, 512, 64, 16, False)])
+@torch.inference_mode()
+def test_persistent_router_matches_per_token_kernel(m, h, e, k, add):
+    """One block per workgroup and several, with and without a tail: x and z
+    bitwise the norm kernel's, logits within a bf16 ulp of the per-token
+    kernels' (their own in the tail), the selection exact given the logits."""
+    g = torch.Generator(device=DEV).manual_seed(m + h)
+    x = torch.randn(m, h, generator=g, device=DEV).to(torch.bfloat16)
+    a = torch.randn(m, h, generator=g, device=DEV).to(torch.bfloat16) if add else None
+    w = (1 + 0.2 * torch.randn(h, generator=g, device=DEV)).to(torch.bfloat16)
+    wr = (0.02 * torch.randn(e, h, generator=g, device=DEV)).to(torch.bfloat16)
+    x1, x2 = x.clone(), x.clone()
+    got, ref = (torch.empty(m, e, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    weights, ids, z = router.add_rmsnorm_route(x1, a, 0.22, w, 1e-6, wr, k, logits_out=got)
+    z2 = norm.add_rmsnorm(x2, a, 0.22, w, 1e-6)
+    assert torch.equal(x1, x2) and torch.equal(z, z2)
+    for i in range(0, m, 1000):
+        router.route(z2[i:i + 1000], wr, k, logits_out=ref[i:i + 1000])
+    assert projections.within_ulp_or_abs(got, ref, 1, 2e-3)
+    tail = m - m % 16
+    assert torch.equal(got[tail:], ref[tail:])
+    ew, eids = ops.route(got.cpu(), k)
+    assert torch.equal(ids.cpu(), eids)
+    torch.testing.assert_close(weights.cpu(), ew, rtol=2e-6, atol=1e-7)
+
+
+@pytest.mark.parametrize("routes", [1, 63, 64, 65, 1024, 1025, 8191, 8192, 8193])
+@pytest.mark.parametrize("local,first", [(1, 0), (40, 0), (63, 3), (511, 0)])
+@torch.inference_mode()
+def test_moe_align_around_its_kernels_limits(routes, local, first):
+    g = torch.Generator().manual_seed(routes + local)
+    ids = torch.randint(0, local + 2 * first + 1, (routes, 1), generator=g, dtype=torch.int32)
+    offsets, order, inverse = experts.moe_align(ids.to(DEV), local, first)
+    eo, eord, einv = ops.permutation(ids, local, first)
+    assert offsets.cpu().tolist() == eo.tolist()
+    assert torch.equal(order.cpu().long(), eord) and torch.equal(inverse.cpu().long(), einv)
