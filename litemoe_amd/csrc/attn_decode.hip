@@ -427,25 +427,49 @@ decode_kernel(const bf16 *__restrict__ q, int64_t qs0, int64_t qs1, bf16 *__rest
   }
 }
 
-// grid (q_heads, batch), one thread per channel.
+// grid (q_heads, batch), one thread per channel. The partials of kCombineBatch
+// splits (4 or 16 by the split count) are requested together (clamped and masked, so none
+// waits behind the row's length): one load round trip up to that many splits
+// instead of two per split. 3 rows, 16 q heads, 15 splits, in the decode graph:
+// 6.9 -> 2.9 us.
+template <int kCombineBatch>
 __global__ void __launch_bounds__(kD)
 decode_combine_kernel(const int32_t *__restrict__ used, int q_heads, int64_t capacity, int max_len,
                       int chunk, int splits, Partial part, bf16 *__restrict__ out, int out_mb) {
   const int hq = blockIdx.x;
   const int64_t b = blockIdx.y;
   const int c = threadIdx.x;
+  const int64_t base = ((int64_t)b * q_heads + hq) * splits;
+  float ms[kCombineBatch], ls[kCombineBatch], os[kCombineBatch];
+  auto load = [&](int s0) {
+#pragma unroll
+    for (int i = 0; i < kCombineBatch; ++i) ms[i] = part.m[base + min(s0 + i, splits - 1)];
+#pragma unroll
+    for (int i = 0; i < kCombineBatch; ++i) {
+      ls[i] = part.l[base + min(s0 + i, splits - 1)];
+      os[i] = part.o[(base + min(s0 + i, splits - 1)) * kD + c];
+    }
+  };
+  load(0);
   int n = used[b];
   n = min(n, max_len);
   n = (int)min((int64_t)n, capacity);
   const int valid = n > 0 ? min(splits, (n + chunk - 1) / chunk) : 0;
-  const int64_t base = ((int64_t)b * q_heads + hq) * splits;
   float mx = -INFINITY;
-  for (int s = 0; s < valid; ++s) mx = fmaxf(mx, part.m[base + s]);
+#pragma unroll
+  for (int i = 0; i < kCombineBatch; ++i) mx = fmaxf(mx, i < valid ? ms[i] : -INFINITY);
+  for (int s = kCombineBatch; s < valid; ++s) mx = fmaxf(mx, part.m[base + s]);
   float lsum = 0.f, o = 0.f;
-  for (int s = 0; s < valid; ++s) {
-    const float f = merge_factor(part.m[base + s], mx);
-    lsum += part.l[base + s] * f;
-    o += part.o[(base + s) * kD + c] * f;
+  for (int s0 = 0; s0 < valid; s0 += kCombineBatch) {
+    if (s0) load(s0);
+#pragma unroll
+    for (int i = 0; i < kCombineBatch; ++i) {
+      // an empty split's partials were never written: selected away, not scaled
+      const bool live = s0 + i < valid;
+      const float f = live ? merge_factor(ms[i], mx) : 0.f;
+      lsum += live ? ls[i] * f : 0.f;
+      o += live ? os[i] * f : 0.f;
+    }
   }
   out[out_index(b, hq, c, q_heads, out_mb)] = (bf16)f32_to_bf16(lsum > 0.f ? o / lsum : 0.f);
 }
@@ -516,7 +540,8 @@ int launch_decode(const void *q, int64_t qs0, int64_t qs1, void *k_cache, void *
   }
   LM_CHECK_LAUNCH();
   if (splits > 1) {
-    decode_combine_kernel<<<dim3((unsigned)q_heads, (unsigned)batch), kD, 0, s>>>(
+    auto combine = splits <= 4 ? decode_combine_kernel<4> : decode_combine_kernel<16>;
+    combine<<<dim3((unsigned)q_heads, (unsigned)batch), kD, 0, s>>>(
         used, (int)q_heads, capacity, (int)max_len, chunk, stride_splits, part, (bf16 *)out,
         out_mb);
     LM_CHECK_LAUNCH();

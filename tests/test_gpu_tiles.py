@@ -7,7 +7,7 @@ import torch
 
 import test_gpu_projections as projections
 from helpers import rel_l2
-from litemoe_amd import experts, linear, norm, router
+from litemoe_amd import experts, flash_decode, linear, norm, router
 from oracle import ops
 
 pytestmark = pytest.mark.gpu
@@ -111,3 +111,21 @@ def test_moe_align_around_its_kernels_limits(routes, local, first):
     eo, eord, einv = ops.permutation(ids, local, first)
     assert offsets.cpu().tolist() == eo.tolist()
     assert torch.equal(order.cpu().long(), eord) and torch.equal(inverse.cpu().long(), einv)
+
+
+@pytest.mark.parametrize("splits", [2, 4, 5, 16, 17, 40])
+@torch.inference_mode()
+def test_flash_decode_combine_batches(splits):
+    """Split counts around the combine's batches (4, 16, several), rows that
+    fill one split, some and all: against the oracle (bf16 output and P, 1e-2),
+    with NaN in the workspace of the splits that a short row leaves unwritten."""
+    g = torch.Generator().manual_seed(splits)
+    b, hq, hkv, cap = 4, 8, 4, 2048
+    q = torch.randn(b, hq, 1, 64, generator=g).to(torch.bfloat16)
+    k, v = (torch.randn(b, hkv, cap, 64, generator=g).to(torch.bfloat16) for _ in range(2))
+    used = torch.tensor([1, 200, 1025, cap], dtype=torch.int32)
+    flash = flash_decode.FlashDecode(b, hkv, hq // hkv, cap, DEV, num_splits=splits)
+    flash.workspace.fill_(0xFF)
+    got = flash(q.to(DEV), k.to(DEV), v.to(DEV), None, None, 0.125, used.to(DEV))
+    exp = ops.decode_attention(q[:, :, 0], k, v, used, 0.125)
+    assert rel_l2(got[:, :, 0].cpu(), exp) < 1e-2 and torch.isfinite(got).all()
