@@ -93,8 +93,19 @@ gemm_kernel(const bf16 *__restrict__ a, int64_t lda, const bf16 *__restrict__ w,
   // registers more and 2% more time); three or more are one array.
   __shared__ __align__(16) char s0[kStages == 2 ? kStage : kStages * kStage];
   __shared__ __align__(16) char s1[kStages == 2 ? kStage : 16];
-  __shared__ int64_t st_pos[kRope ? kTM : 1];  // kRope, kStore == 2: cache position per row
-  __shared__ int st_slot[kRope ? kTM : 1];
+  // kRope, kStore == 2: cache position and slot per row. They live in the
+  // stages behind the staged output tile where there is room (the 192 x 128
+  // tile's two workgroups per CU need all 160 KB for the stages).
+  constexpr int kTileBytes = kTM * kTN * 2, kStageAll = kStages * kStage;
+  constexpr bool kSpare = kRope && kStore == 2 && kStageAll - kTileBytes >= kTM * 12 && kTileBytes >= (int)sizeof(s0);
+  __shared__ int64_t st_pos_own[kRope && !kSpare ? kTM : 1];
+  __shared__ int st_slot_own[kRope && !kSpare ? kTM : 1];
+  [[maybe_unused]] int64_t *st_pos = st_pos_own;
+  [[maybe_unused]] int *st_slot = st_slot_own;
+  if constexpr (kSpare) {
+    st_pos = reinterpret_cast<int64_t *>(s1 + (kTileBytes - (int)sizeof(s0)));
+    st_slot = reinterpret_cast<int *>(st_pos + kTM);
+  }
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int lin = blockIdx.x;
   int tile_m = lin / tiles_n, tile_n = lin % tiles_n;
@@ -331,6 +342,14 @@ gemm_kernel(const bf16 *__restrict__ a, int64_t lda, const bf16 *__restrict__ w,
       }
     }
     __syncthreads();
+    // The rotated q, k, v and the cache rows of a large prefill leave
+    // non-temporal: they would push the operand tiles out of the L2s (the
+    // block of 25k tokens at hidden 1024 346 -> 340 us, of 7584 at 1536 165 ->
+    // 162, of 47k unchanged; A/B on one box).
+    auto store = [&](u32x4 *dst, const u32x4 &word) {
+      if constexpr (kRope && kTM >= 192) __builtin_nontemporal_store(word, dst);
+      else *dst = word;
+    };
 #pragma unroll
     for (int i = 0; i < (kTM * kChunks + 64 * kWaves - 1) / (64 * kWaves); ++i) {
       const int idx = i * 64 * kWaves + threadIdx.x;
@@ -338,7 +357,7 @@ gemm_kernel(const bf16 *__restrict__ a, int64_t lda, const bf16 *__restrict__ w,
       const int row = m0 + rl, col = n0 + c * 8;
       if (rl >= kTM || row >= M || col >= N) continue;
       const u32x4 word = *reinterpret_cast<const u32x4 *>(staged(rl) + ((c ^ (rl & kSw)) << 4));
-      *reinterpret_cast<u32x4 *>(out + (int64_t)row * ldo + col) = word;
+      store(reinterpret_cast<u32x4 *>(out + (int64_t)row * ldo + col), word);
       if constexpr (kRope) {
         const int h = col / 64 - rk.q_heads;  // k heads, then v heads
         const int64_t sp = st_pos[rl];
@@ -346,7 +365,7 @@ gemm_kernel(const bf16 *__restrict__ a, int64_t lda, const bf16 *__restrict__ w,
           const bool is_k = h < rk.kv_heads;
           const int kvh = is_k ? h : h - rk.kv_heads;
           bf16 *dst = (is_k ? rk.kc : rk.vc) + (((int64_t)st_slot[rl] * rk.kv_heads + kvh) * rk.capacity + sp) * 64;
-          *reinterpret_cast<u32x4 *>(dst + col % 64) = word;
+          store(reinterpret_cast<u32x4 *>(dst + col % 64), word);
         }
       }
     }
@@ -462,7 +481,14 @@ int launch_gemm_tiled(const bf16 *a, int64_t lda, const bf16 *w, int64_t ldw, bf
     if (tiles(128, 64) <= 256) return launch_gemm_cfg<128, 64, 4, 1, 3, kRope>;
     if (tiles(64, 128) <= 512) return launch_gemm_cfg<64, 128, 2, 2, 3, kRope>;
     if (tiles(128, 128) <= 512) return launch_gemm_cfg<128, 128, 4, 2, 2, kRope>;
-    if (tiles(192, 128) <= 512) return launch_gemm_cfg<192, 128, 4, 2, 2, kRope>;
+    // Beyond one round, 256 x 256 tiles take less time per output unless their
+    // last round is mostly empty: below three quarters of the slots that their
+    // rounds have, 192 x 128 (two per CU) are faster (7584 x 2560 x 1536 64.4
+    // against 70.9 us at 0.59, 10000 x 2560 78.5 against 77.7 at 0.78; 20000 x
+    // 1024 x 1024 42.9 against 53.2 at 0.62).
+    const int64_t large = tiles(256, 256);
+    if (tiles(192, 128) <= 512 || 4 * large < 3 * align_up(large, 256))
+      return launch_gemm_cfg<192, 128, 4, 2, 2, kRope>;
     return launch_gemm_cfg<256, 256, 4, 4, 2, kRope>;
   };
   return pick()(a, lda, w, ldw, out, ldo, M, N, K, stream, rope);
