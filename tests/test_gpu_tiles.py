@@ -129,3 +129,11 @@ def test_flash_decode_combine_batches(splits):
     got = flash(q.to(DEV), k.to(DEV), v.to(DEV), None, None, 0.125, used.to(DEV))
     exp = ops.decode_attention(q[:, :, 0], k, v, used, 0.125)
     assert rel_l2(got[:, :, 0].cpu(), exp) < 1e-2 and torch.isfinite(got).all()
+
+
+@pytest.mark.parametrize("m,h,i,e,k", [(264, 1536, 512, 40, 8), (265, 1536, 512, 40, 8), (511, 384, 128, 7, 5),
+                                       (2113, 128, 128, 3, 1)])
+@torch.inference_mode()
+def test_expert_gemm_line_matches_oracle(m, h, i, e, k):
+    """Both sides of the route count from which the grouped GEMMs run."""
+    test_expert_gemm_tiles_match_oracle(m, h, i, e, k)
