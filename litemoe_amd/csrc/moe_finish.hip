@@ -1,7 +1,8 @@
 // Weighted combine of route outputs (the moe_finish contract):
 //   out[t] = bf16( sum_{j in ascending logical(ids[t,j])*K + j}
 //                  bf16(bf16(y[row(t,j)]) * bf16(scales[t,j])) )   (fp32 sum)
-// Non-owned routes are skipped and their rows never read.
+// Non-owned routes are skipped: nothing of their rows enters the sum (and
+// behind an inverse map, which need not name them, they are never read).
 // Reference: litemoe/moe_finish.py:7-31 (`_finish`), :34-57 (`finish`).
 #include "internal.h"
 
@@ -11,26 +12,48 @@ namespace {
 constexpr int kMaxK = 8;
 
 // grid (tokens, column blocks); each thread owns kCols consecutive columns.
-template <int kCols>
+template <int kCols, bool kDirect = false>
 __global__ void __launch_bounds__(256)
 finish_kernel(const bf16 *__restrict__ y, const int32_t *__restrict__ ids,
               const int32_t *__restrict__ inverse, const float *__restrict__ scales,
               const int64_t *__restrict__ logical, bf16 *__restrict__ out, int hidden, int topk,
               int64_t rank, int64_t count) {
   const int64_t t = blockIdx.x;
-  const int c0 = (blockIdx.y * 256 + threadIdx.x) * kCols;
-  if (c0 >= hidden) return;
+  int c0 = (blockIdx.y * 256 + threadIdx.x) * kCols;
+  // kDirect reads lanes 0 .. topk - 1 of every wave, so threads past the row
+  // stay, on its last columns, up to the store.
+  const bool live = c0 < hidden;
+  if (!kDirect && !live) return;
+  if constexpr (kDirect) c0 = min(c0, hidden - kCols);
   // Rank of each branch under the key logical*K + j (keys are distinct:
   // j differs). A route that is not owned adds nothing wherever it ranks, so
   // its key uses the raw id and the map is read for owned ids only (an id
   // outside every rank's range never indexes it). The workgroup's threads
   // share the token, so ids, keys and ranks are uniform (scalar registers)
   // and the ordered sum below branches uniformly.
+  // kDirect: lane j loads route j's id and scale, and every route row is
+  // requested with them (a row that is not owned is loaded and its values
+  // dropped), so the kernel waits on memory once instead of once per scalar
+  // load and branch (the operator of 700 tokens, hidden 1536, with the norm
+  // behind it: 90.4 -> 88.2 us).
+  u32x4 yv[kDirect ? kMaxK : 1];
+  int id_lane = 0;
+  float sc_lane = 0.f;
+  if constexpr (kDirect) {
+    const int64_t rl = t * topk + min((int)(threadIdx.x % kWave), topk - 1);
+    id_lane = ids[rl];
+    sc_lane = scales[rl];
+#pragma unroll
+    for (int j = 0; j < kMaxK; ++j)
+      yv[j] = *reinterpret_cast<const u32x4 *>(y + (t * topk + min(j, topk - 1)) * hidden + c0);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   int64_t key[kMaxK];
 #pragma unroll
   for (int j = 0; j < kMaxK; ++j) {
     if (j < topk) {
-      const int64_t e = __builtin_amdgcn_readfirstlane(ids[t * topk + j]);
+      const int64_t e = kDirect ? __builtin_amdgcn_readlane(id_lane, j)
+                                : __builtin_amdgcn_readfirstlane(ids[t * topk + j]);
       const bool owned = e - rank * count >= 0 && e - rank * count < count;
       key[j] = (logical && owned ? logical[e] : e) * topk + j;
     } else {
@@ -52,6 +75,16 @@ finish_kernel(const bf16 *__restrict__ y, const int32_t *__restrict__ ids,
 #pragma unroll
   for (int j = 0; j < kMaxK; ++j) {
     const int64_t r = t * topk + j;
+    if constexpr (kDirect) {
+      const int64_t e = (int64_t)__builtin_amdgcn_readlane(id_lane, j) - rank * count;
+      const bool use = j < topk && e >= 0 && e < count;
+      const float s = round_bf16(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(sc_lane), j)));
+      float v[8];
+      unpack8(yv[j], v);
+#pragma unroll
+      for (int c = 0; c < 8; ++c) contrib[j][c] = use ? round_bf16(v[c] * s) : 0.f;
+      continue;
+    }
     const int64_t e = j < topk ? (int64_t)ids[r] - rank * count : -1;
     const bool use = j < topk && e >= 0 && e < count;
     const float s = use ? round_bf16(scales[r]) : 0.f;
@@ -83,6 +116,7 @@ finish_kernel(const bf16 *__restrict__ y, const int32_t *__restrict__ ids,
       }
     }
   }
+  if (!live) return;
   bf16 *o = out + t * hidden + c0;
   if constexpr (kCols == 8) {
     u32x4 w;
@@ -236,8 +270,9 @@ int launch_finish(const bf16 *y, const int32_t *ids, const int32_t *inverse, con
   if (tokens == 0) return LM_OK;
   if (hidden % 8 == 0) {
     const dim3 grid((unsigned)tokens, (unsigned)cdiv(hidden, 256 * 8));
-    finish_kernel<8><<<grid, 256, 0, stream>>>(y, ids, inverse, scales, logical, out, (int)hidden,
-                                               (int)topk, rank, count);
+    auto kernel = inverse ? finish_kernel<8> : finish_kernel<8, true>;
+    kernel<<<grid, 256, 0, stream>>>(y, ids, inverse, scales, logical, out, (int)hidden, (int)topk, rank,
+                                     count);
   } else {
     const dim3 grid((unsigned)tokens, (unsigned)cdiv(hidden, 256));
     finish_kernel<1><<<grid, 256, 0, stream>>>(y, ids, inverse, scales, logical, out, (int)hidden,

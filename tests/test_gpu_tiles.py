@@ -7,7 +7,7 @@ import torch
 
 import test_gpu_projections as projections
 from helpers import rel_l2
-from litemoe_amd import experts, flash_decode, linear, norm, router
+from litemoe_amd import _lib, experts, flash_decode, linear, norm, router
 from oracle import ops
 
 pytestmark = pytest.mark.gpu
@@ -137,3 +137,26 @@ def test_flash_decode_combine_batches(splits):
 def test_expert_gemm_line_matches_oracle(m, h, i, e, k):
     """Both sides of the route count from which the grouped GEMMs run."""
     test_expert_gemm_tiles_match_oracle(m, h, i, e, k)
+
+
+@pytest.mark.parametrize("batch,topk,hidden,rank,remap", [
+    (3, 8, 8, 0, False), (5, 3, 1544, 0, True), (4, 8, 4104, 1, False), (700, 8, 1536, 0, False)])
+@torch.inference_mode()
+def test_finish_in_route_order(batch, topk, hidden, rank, remap):
+    """lm_moe_finish without an order (rows in route order), bit-exact against
+    the oracle: waves with one column in the row, routes of another rank (NaN
+    rows) and a logical map."""
+    g = torch.Generator().manual_seed(batch + hidden)
+    count = 8
+    ids = torch.stack([torch.randperm(2 * count, generator=g)[:topk] for _ in range(batch)]).int()
+    y = torch.randn(batch * topk, hidden, generator=g).to(torch.bfloat16)
+    y[(ids.flatten() < rank * count) | (ids.flatten() >= (rank + 1) * count)] = float("nan")
+    scales = torch.softmax(torch.randn(batch, topk, generator=g), -1)
+    logical = torch.randperm(2 * count, generator=g) if remap else None
+    out = torch.full((batch + 1, hidden), 7.0, dtype=torch.bfloat16, device=DEV)
+    d = [t.to(DEV) for t in (y, ids, scales)]
+    lg = None if logical is None else logical.to(DEV)
+    _lib.call("lm_moe_finish", d[0].data_ptr(), d[1].data_ptr(), None, d[2].data_ptr(), _lib.ptr(lg), out.data_ptr(),
+              batch, hidden, topk, rank, count, None, 0, _lib.stream(out.device))
+    assert torch.equal(out[:batch].cpu(), ops.finish(y, ids, scales, rank, count, logical))
+    assert (out[batch] == 7).all()
