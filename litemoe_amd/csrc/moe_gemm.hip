@@ -38,6 +38,7 @@ enum RouteMode : int {
   kBlocks = 0,        // lm_moe_align blocks; weights after the block lookup
   kScanLazy = 1,      // scan of topk_ids; weights only once routes are found
   kScanPrefetch = 2,  // scan of topk_ids; weights issued before the scan
+  kScanFew = 3,       // at most kFewRoutes routes: each wave finds them itself, then the weights
 };
 
 // Block b of the per-expert blocks of block_rows routes.
@@ -117,6 +118,45 @@ __device__ int scan_ids(const ScanIds &s, int e, int *list, int *wave_count) {
   }
   __syncthreads();
   return total;
+}
+
+// Route collection for a few routes (at most kFewRoutes), by each wave for
+// itself: every lane loads kFewIters ids, ballots find the expert's routes,
+// and the wave writes them in ascending order into a list of its own. No
+// barrier, and an expert without routes (most of them, for a few tokens)
+// is known after the one load.
+constexpr int kFewIters = 4, kFewRoutes = kFewIters * kWave;
+static_assert(kWaves * kFewRoutes <= kScanList, "the waves' lists share the scan's LDS");
+
+struct FewRoutes {
+  uint64_t mask[kFewIters];
+  int count;
+};
+
+__device__ __forceinline__ FewRoutes find_few(const int32_t *__restrict__ ids, int routes, int e) {
+  const int lane = threadIdx.x % kWave;
+  int id[kFewIters];
+#pragma unroll
+  for (int it = 0; it < kFewIters; ++it) id[it] = ids[min(it * kWave + lane, routes - 1)];
+  FewRoutes f;
+  f.count = 0;
+#pragma unroll
+  for (int it = 0; it < kFewIters; ++it) {
+    f.mask[it] = __ballot(id[it] == e && it * kWave + lane < routes);
+    f.count += __popcll(f.mask[it]);
+  }
+  return f;
+}
+
+__device__ __forceinline__ void list_few(const FewRoutes &f, int *list) {
+  const int lane = threadIdx.x % kWave;
+  int offset = 0;
+#pragma unroll
+  for (int it = 0; it < kFewIters; ++it) {
+    if ((f.mask[it] >> lane) & 1) list[offset + __popcll(f.mask[it] & ((1ull << lane) - 1ull))] = it * kWave + lane;
+    offset += __popcll(f.mask[it]);
+  }
+  __builtin_amdgcn_wave_barrier();  // LDS keeps a wave's order: its reads follow
 }
 
 constexpr int kXcdCount = 8;
@@ -252,7 +292,10 @@ gate_up_kernel(const bf16 *__restrict__ x, const bf16 *__restrict__ w13,
 // runs without the row-block loop. That keeps a wave within 128 registers up
 // to hidden 1536, so four workgroups share a CU: 1024 of the decode step's
 // 1280 weight tiles (Granite-3B shape) are in flight at once instead of 768.
-template <int KS, bool kPacked>
+// kFew: at most kFewRoutes routes, found by find_few, the weights requested
+// only by the workgroups of experts that have some (a call of a few tokens
+// leaves most experts out).
+template <int KS, bool kPacked, bool kFew = false>
 __global__ void __launch_bounds__(kThreads, KS <= 12 ? 4 : 2)
 gate_up_scan_kernel(const bf16 *__restrict__ x, const bf16 *__restrict__ w13,
                     const int32_t *__restrict__ ids, int routes, int topk, int hidden, int inter,
@@ -262,7 +305,7 @@ gate_up_scan_kernel(const bf16 *__restrict__ x, const bf16 *__restrict__ w13,
   if (zero_counters && blockIdx.x == 0 && blockIdx.y == 0 && (int)threadIdx.x < counters)
     zero_counters[threadIdx.x] = 0;
   __shared__ float red[kWaves][2][4][kWave];
-  __shared__ int list[kScanList];
+  __shared__ int list_lds[kScanList];
   __shared__ int wave_count[kWaves];
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int col = lane % 16, grp = lane / 16;
@@ -274,16 +317,30 @@ gate_up_scan_kernel(const bf16 *__restrict__ x, const bf16 *__restrict__ w13,
   const bf16 *wg = w13 + wofs<kPacked>(rg, kbase, hidden);
   const bf16 *wu = w13 + wofs<kPacked>(rg + inter, kbase, hidden);
   u32x4 bg[KS], bu[KS], a[KS];
-  const ScanIds scan = load_ids(ids, routes);
-  __builtin_amdgcn_sched_barrier(0);  // ids first: the scan waits for them only
+  auto load_weights = [&]() {
 #pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    bg[s] = load16_stream(wg + s * wstep<kPacked>());
-    bu[s] = load16_stream(wu + s * wstep<kPacked>());
+    for (int s = 0; s < KS; ++s) {
+      bg[s] = load16_stream(wg + s * wstep<kPacked>());
+      bu[s] = load16_stream(wu + s * wstep<kPacked>());
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int n;
+  int *list = list_lds;
+  if constexpr (kFew) {
+    const FewRoutes few = find_few(ids, routes, e);
+    n = few.count;
+    if (n == 0) return;
+    load_weights();
+    list += wave * kFewRoutes;
+    list_few(few, list);
+  } else {
+    const ScanIds scan = load_ids(ids, routes);
+    __builtin_amdgcn_sched_barrier(0);  // ids first: the scan waits for them only
+    load_weights();
+    n = scan_ids(scan, e, list, wave_count);
+    if (n == 0) return;
   }
-  __builtin_amdgcn_sched_barrier(0);
-  const int n = scan_ids(scan, e, list, wave_count);
-  if (n == 0) return;
   auto block = [&](int rb) {
     const bf16 *xr = x + (int64_t)(list[min(rb + col, n - 1)] / topk) * hidden + kbase;
 #pragma unroll
@@ -570,14 +627,16 @@ __device__ void combine_tile(const TileCombine &c, const bf16 *__restrict__ term
 // per wave, inter = KS * 32 * kWaves); its activation loads are issued back
 // to back. Same MFMA order and wave-order sum as down_kernel, hence the same
 // bits. kFin: the combine fused in (TileCombine; NT == 4, 64-column tiles).
-template <int KS, int NT, bool kPacked, int kFin = 0>
+// kFew: as in gate_up_scan_kernel.
+template <int KS, int NT, bool kPacked, int kFin = 0, bool kFew = false>
 __global__ void __launch_bounds__(kThreads)
 down_scan_kernel(const bf16 *__restrict__ act, const bf16 *__restrict__ w2,
                  const int32_t *__restrict__ ids, int routes, int hidden, int inter,
                  bf16 *__restrict__ y, TileCombine fin) {
+  static_assert(kFin == 0 || !kFew, "the fused combine takes the scan");
   static_assert(kFin == 0 || NT == 4, "the fused combine works on 64-column tiles");
   __shared__ float red[kWaves][NT][4][kWave];
-  __shared__ int list[kScanList];
+  __shared__ int list_lds[kScanList];
   __shared__ int wave_count[kWaves];
   __shared__ int last_flag;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
@@ -588,16 +647,30 @@ down_scan_kernel(const bf16 *__restrict__ act, const bf16 *__restrict__ w2,
   const int kbase = wave * KS * 32 + grp * 8;
   const int64_t r0 = (int64_t)e * hidden + n0 + col;
   u32x4 b[NT][KS], a[KS];
-  const ScanIds scan = load_ids(ids, routes);
-  __builtin_amdgcn_sched_barrier(0);  // ids first: the scan waits for them only
+  auto load_weights = [&]() {
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const bf16 *wt = w2 + wofs<kPacked>(r0 + 16 * t, kbase, inter);
+    for (int t = 0; t < NT; ++t) {
+      const bf16 *wt = w2 + wofs<kPacked>(r0 + 16 * t, kbase, inter);
 #pragma unroll
-    for (int s = 0; s < KS; ++s) b[t][s] = load16_stream(wt + s * wstep<kPacked>());
+      for (int s = 0; s < KS; ++s) b[t][s] = load16_stream(wt + s * wstep<kPacked>());
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int n;
+  int *list = list_lds;
+  if constexpr (kFew) {
+    const FewRoutes few = find_few(ids, routes, e);
+    n = few.count;
+    if (n == 0) return;
+    load_weights();
+    list += wave * kFewRoutes;
+    list_few(few, list);
+  } else {
+    const ScanIds scan = load_ids(ids, routes);
+    __builtin_amdgcn_sched_barrier(0);  // ids first: the scan waits for them only
+    load_weights();
+    n = scan_ids(scan, e, list, wave_count);
   }
-  __builtin_amdgcn_sched_barrier(0);
-  const int n = scan_ids(scan, e, list, wave_count);
   auto block = [&](int rb) {
     const bf16 *ar = act + (int64_t)list[min(rb + col, n - 1)] * inter + kbase;
 #pragma unroll
@@ -683,7 +756,9 @@ bool ks_ok(int64_t n) {
 // Weight tiles are prefetched before the route scan when an empty expert is
 // unlikely (>= 4 routes per expert on average).
 int route_mode(bool scan, int64_t routes, int64_t experts) {
-  return !scan ? kBlocks : (routes >= 4 * experts ? kScanPrefetch : kScanLazy);
+  if (!scan) return kBlocks;
+  if (routes >= 4 * experts) return kScanPrefetch;
+  return routes <= kFewRoutes ? kScanFew : kScanLazy;
 }
 
 }  // namespace
@@ -719,6 +794,9 @@ int launch_gate_up_t(const bf16 *x, const bf16 *w13, const int32_t *offsets, con
   case KS:                                                                                      \
     if (mode == kScanPrefetch)                                                                  \
       gate_up_scan_kernel<KS, kPacked><<<grid, kThreads, 0, stream>>>(x, w13, ids, (int)routes,          \
+          (int)topk, (int)hidden, (int)inter, act, nullptr, 0);                                 \
+    else if (mode == kScanFew)                                                                  \
+      gate_up_scan_kernel<KS, kPacked, true><<<grid, kThreads, 0, stream>>>(x, w13, ids, (int)routes,    \
           (int)topk, (int)hidden, (int)inter, act, nullptr, 0);                                 \
     else if (mode == kScanLazy)                                                                 \
       gate_up_kernel<KS, kScanLazy, kPacked><<<grid, kThreads, 0, stream>>>(x, w13, offsets, sorted,     \
@@ -766,13 +844,27 @@ int launch_down_t(const bf16 *act, const bf16 *w2, const int32_t *offsets, const
         break;
     }
   }
+  if (mode == kScanFew && inter <= 8 * 128) {
+    switch (inter / 128) {
+#define X(KS)                                                                                  \
+  case KS:                                                                                     \
+    down_scan_kernel<KS, 2, kPacked, 0, true><<<grid, kThreads, 0, stream>>>(                           \
+        act, w2, ids, (int)routes, (int)hidden, (int)inter, y, TileCombine{});                 \
+    LM_CHECK_LAUNCH();                                                                         \
+    return LM_OK;
+      X(1) X(2) X(3) X(4) X(6) X(8)
+#undef X
+      default:
+        break;
+    }
+  }
   switch (inter / 128) {
 #define X(KS)                                                                                  \
   case KS:                                                                                     \
     if (mode == kScanPrefetch)                                                                 \
       down_kernel<KS, kScanPrefetch, kPacked><<<grid, kThreads, 0, stream>>>(act, w2, offsets, sorted,  \
           ids, (int)routes, (int)hidden, (int)inter, (int)experts, bm, y);                     \
-    else if (mode == kScanLazy)                                                                \
+    else if (mode == kScanLazy || mode == kScanFew)                                            \
       down_kernel<KS, kScanLazy, kPacked><<<grid, kThreads, 0, stream>>>(act, w2, offsets, sorted, ids, \
           (int)routes, (int)hidden, (int)inter, (int)experts, bm, y);                          \
     else                                                                                       \

@@ -160,3 +160,24 @@ def test_finish_in_route_order(batch, topk, hidden, rank, remap):
               batch, hidden, topk, rank, count, None, 0, _lib.stream(out.device))
     assert torch.equal(out[:batch].cpu(), ops.finish(y, ids, scales, rank, count, logical))
     assert (out[batch] == 7).all()
+
+
+@pytest.mark.parametrize("m,h,i,e,k,hot", [
+    (1, 1024, 512, 32, 8, False), (5, 1536, 512, 40, 8, False), (8, 256, 128, 17, 8, True),
+    (31, 512, 256, 64, 8, True), (32, 128, 1024, 65, 8, False), (33, 128, 128, 100, 8, True)])
+@pytest.mark.parametrize("packed", [False, True])
+@torch.inference_mode()
+def test_few_routes_equal_block_path(m, h, i, e, k, hot, packed):
+    """Calls below four routes per expert, to 256 routes (each wave finds its
+    expert's routes) and past them: the bits of the aligned-block path, with
+    experts of none, some and more than 16 and 32 routes."""
+    g = torch.Generator().manual_seed(m + e)
+    x = torch.randn(m, h, generator=g).to(torch.bfloat16).to(DEV)
+    w1 = (torch.randn(e, 2 * i, h, generator=g) * 0.05).to(torch.bfloat16).to(DEV)
+    w2 = (torch.randn(e, h, i, generator=g) * 0.05).to(torch.bfloat16).to(DEV)
+    ids = torch.stack([torch.randperm(e, generator=g)[:k] for _ in range(m)]).int()
+    if hot:
+        ids[:, 0] = e - 1  # also as a repeated id
+    ids = ids.to(DEV)
+    w = experts.pack_expert_weights(w1, w2) if packed else (w1, w2)
+    assert torch.equal(experts.moe_routes(x, *w, ids, packed=packed), experts.moe_routes(x, w1, w2, ids, block_rows=16))
