@@ -754,7 +754,10 @@ bool ks_ok(int64_t n) {
 }
 
 // Weight tiles are prefetched before the route scan when an empty expert is
-// unlikely (>= 4 routes per expert on average).
+// unlikely (>= 4 routes per expert on average): four layers at hidden 1536, 40
+// experts, us: 24 rows 157.5 against 164 without the prefetch (167 and 170
+// with half of the routes on four experts), 10 rows 158 against 152 (156 and
+// 144 with them).
 int route_mode(bool scan, int64_t routes, int64_t experts) {
   if (!scan) return kBlocks;
   if (routes >= 4 * experts) return kScanPrefetch;

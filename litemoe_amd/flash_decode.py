@@ -20,11 +20,24 @@ from .linear import FragRows
 
 
 def default_splits(batch, kv_heads, maximum, target_workgroups=512, min_keys=256, max_splits=16):
-    """Split the key range only as far as needed to give the GPU about
-    ``target_workgroups`` (batch * kv_heads * splits) workgroups, keeping at
-    least ``min_keys`` keys per split; one split needs no combine pass."""
-    want = math.ceil(target_workgroups / max(1, batch * kv_heads))
-    return max(1, min(max_splits, want, maximum // min_keys))
+    """Key-range splits of ``batch * kv_heads`` (row, head) pairs over contexts
+    up to ``maximum``.
+
+    Up to half of ``target_workgroups`` pairs (one workgroup of eight waves
+    per CU) the splits fill that half and no more: a second workgroup on a CU
+    shares its load rate, and every split adds a prologue and partials to
+    combine. Measured as the attention block of a decode graph, us per layer,
+    against splits for the whole target: 24 rows x 8 heads to 2000 keys 31.3
+    (1 split) and 36.9 (3); 10 rows 24.7 (3) and 29.5 (7); 3 rows to 4001 keys
+    21.2 (10) and 23.2 (15); 32 rows to 1500 27.6 (1) and 30.2 (2). Beyond it,
+    the splits bring the workgroups to the target (40 rows to 4000 keys 70.8
+    with 2 splits, 73.5 with 1). A split keeps at least ``min_keys`` keys, and
+    contexts below three times that are not split, since their combine costs
+    more than the shorter stream saves (one row, 512 keys: 16.4 and 17.4)."""
+    pairs, half = max(1, batch * kv_heads), target_workgroups // 2
+    want = half // pairs if pairs <= half else math.ceil(target_workgroups / pairs)
+    longest = maximum // min_keys if maximum >= 3 * min_keys else 1
+    return max(1, min(max_splits, want, longest))
 
 
 class FlashDecode:
