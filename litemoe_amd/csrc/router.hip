@@ -714,9 +714,12 @@ batched_router_kernel(bf16 *__restrict__ x, const bf16 *__restrict__ a, float al
 // bytes: a fragment's 16 rows fall on 16 bank groups) instead of being read
 // back from L2; and the next block's row is in flight from the moment the norm
 // has taken this block's, so HBM streams under the logits and the selection
-// instead of alternating with them. The last tokens % 16 are routed beside the
-// blocks in the per-token kernels' order, so there is no tail launch; the
-// blocks' x, z and logits are bitwise batched_router_kernel's. The stream bounds it: 577 MB at 46,990
+// instead of alternating with them. The last tokens % 16 are routed in the
+// per-token kernels' order, one per workgroup, by those whose next block they
+// would be, so there is no tail launch (all of them on one workgroup held the
+// launch back: 1039 tokens of hidden 1536 19.3 -> 11.9 us, 8191 tokens 35.1 ->
+// 29.4, 1039 of hidden 1024 13.9 -> 8.7; 46,990 121.0 -> 120.6); the blocks'
+// x, z and logits are bitwise batched_router_kernel's. The stream bounds it: 577 MB at 46,990
 // tokens of hidden 1536, 40 experts, in 121 us (4.8 TB/s; a large copy
 // reaches 4.9) against 162 us for batched_router_kernel and its tail launch;
 // 2000 tokens 35 -> 13 us; hidden 1024, 32 experts, 46,990 tokens 107 -> 79
@@ -751,7 +754,11 @@ persistent_router_kernel(bf16 *__restrict__ x, const bf16 *__restrict__ a, float
   const int tr = lane % 16, kg = lane / 16;
   const int kq = wave % kBatchWaves, nt = wave / kBatchWaves;  // nt >= NT: no logits
   const int64_t blocks = tokens / kPersistRows;  // whole blocks
-  int64_t row = (int64_t)blockIdx.x * kPersistRows + wave;
+  // the tail token of this workgroup, if below tail (one each, behind the blocks)
+  const int tail = (int)(tokens % kPersistRows), grid = (int)gridDim.x;
+  const int tail_at = ((int)blockIdx.x + grid - (int)(blocks % grid)) % grid;
+  const int64_t tail_row = blocks * kPersistRows + tail_at;
+  int64_t row = blockIdx.x < blocks ? (int64_t)blockIdx.x * kPersistRows + wave : tail_row;
   const int64_t stride = (int64_t)gridDim.x * kPersistRows;
   u32x4 xv[NVL], av[NVL];
   batch_load_row<NVL, kAdd>(x, a, min(row, tokens - 1), xv, av);
@@ -814,45 +821,45 @@ persistent_router_kernel(bf16 *__restrict__ x, const bf16 *__restrict__ a, float
     select_topk_lanes(logit[wave], scratch[wave], lane, n_experts, k, renormalize, tw + row * topk,
                       tid + row * topk);
   }
-  // The last tokens % 16: the workgroup whose next block they would be norms a
-  // token per wave and then takes a gate row per wave over all of them, the
-  // logits in the per-token kernels' order (gate_round).
-  const int tail = (int)(tokens % kPersistRows);
-  if (tail == 0 || blockIdx.x != blocks % gridDim.x) return;
-  row = blocks * kPersistRows + wave;
-  if (wave < tail) {
-    batch_load_row<NVL, kAdd>(x, a, row, xv, av);
-    u32x4 *zrow = zs + wave * kPitch;
+  // A tail token: wave 0 norms it while each wave's gate rows load, and the
+  // logits are summed in the per-token kernels' order (gate_round).
+  if (tail_at >= tail) return;
+  u32x4 gw[NT][NVL];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int i = 0; i < NVL; ++i)
+      gw[n][i] = reinterpret_cast<const u32x4 *>(wr)[(int64_t)min(wave + n * kPersistWaves, experts - 1) * kNvec +
+                                                     lane + i * kWave];
+  if (wave == 0) {
+    if (blockIdx.x < blocks) batch_load_row<NVL, kAdd>(x, a, tail_row, xv, av);
     if constexpr (kNorm) {
       u32x4 gv[NVL];
 #pragma unroll
       for (int i = 0; i < NVL; ++i) gv[i] = gs[lane + i * kWave];
-      batch_norm_row<NVL, kAdd>(x, alpha, gv, eps, z, row, xv, av, zrow);
+      batch_norm_row<NVL, kAdd>(x, alpha, gv, eps, z, tail_row, xv, av, zs);
     } else {
 #pragma unroll
-      for (int i = 0; i < NVL; ++i) zrow[lane + i * kWave] = xv[i];
+      for (int i = 0; i < NVL; ++i) zs[lane + i * kWave] = xv[i];
     }
   }
-  __syncthreads();  // (also: every wave has selected from logit)
-  for (int e = wave; e < experts; e += kPersistWaves) {
-    u32x4 gw[NVL];
+  __syncthreads();  // (also: wave 0 has selected from logit[0])
 #pragma unroll
-    for (int i = 0; i < NVL; ++i) gw[i] = reinterpret_cast<const u32x4 *>(wr)[(int64_t)e * kNvec + lane + i * kWave];
-    for (int r = 0; r < tail; ++r) {
-      float acc = 0.f;
+  for (int n = 0; n < NT; ++n) {
+    const int e = wave + n * kPersistWaves;
+    float acc = 0.f;
 #pragma unroll
-      for (int i = 0; i < NVL; ++i) acc = dot8_bf16_acc(zs[r * kPitch + lane + i * kWave], gw[i], acc);
-      const uint32_t h = f32_to_bf16(wave_sum(acc));
-      if (lane == 0) {
-        logit[r][e] = bf16_to_f32(h);
-        if (logits_out) logits_out[(blocks * kPersistRows + r) * experts + e] = (bf16)h;
-      }
+    for (int i = 0; i < NVL; ++i) acc = dot8_bf16_acc(zs[lane + i * kWave], gw[n][i], acc);
+    const uint32_t h = f32_to_bf16(wave_sum(acc));
+    if (lane == 0 && e < experts) {
+      logit[0][e] = bf16_to_f32(h);
+      if (logits_out) logits_out[tail_row * experts + e] = (bf16)h;
     }
   }
   __syncthreads();
-  if (wave < tail)
-    select_topk_lanes(logit[wave], scratch[wave], lane, experts, topk, renormalize, tw + row * topk,
-                      tid + row * topk);
+  if (wave == 0)
+    select_topk_lanes(logit[0], scratch[0], lane, experts, topk, renormalize, tw + tail_row * topk,
+                      tid + tail_row * topk);
 }
 
 // Routes every token with persistent_router_kernel, or the first
@@ -868,7 +875,7 @@ int64_t launch_batched_router(int64_t tokens, int64_t hidden, bf16 *x, const bf1
   if (tokens < kBatchRouterMinTokens || !nv || experts > kWave || experts <= 16) return 0;
 #define LM_PERSIST_ROUTER(NVL, NT)                                                               \
   if (nv == NVL && (experts + 15) / 16 == NT) {                   \
-    const dim3 pgrid((unsigned)std::min(cdiv(tokens, kPersistRows), kPersistGrid));     \
+    const dim3 pgrid((unsigned)std::min(tokens / kPersistRows + tokens % kPersistRows, kPersistGrid));     \
     persistent_router_kernel<NVL, NT, kNorm, kAdd><<<pgrid, kPersistThreads, 0, s>>>(            \
         x, a, alpha, nw, eps, z, wr, tokens, experts, topk, renormalize, logits_out, tw, tid);   \
     return tokens;                                                                               \
