@@ -25,9 +25,11 @@ constexpr int64_t wstep() { return kPacked ? 64 * 8 : 32; }
 
 // moe_finish.hip: combine of route outputs (see lm_moe_finish).
 // inverse: sorted position of each route, or nullptr when y is in route order.
+// y_readable: y is memory of tokens*topk rows that nothing else writes, so rows
+// of routes that are not owned may be loaded (and dropped); else they are not.
 int launch_finish(const bf16 *y, const int32_t *ids, const int32_t *inverse, const float *scales,
                   const int64_t *logical, bf16 *out, int64_t tokens, int64_t hidden, int64_t topk,
-                  int64_t rank, int64_t count, hipStream_t stream);
+                  int64_t rank, int64_t count, bool y_readable, hipStream_t stream);
 
 // moe_gemm.hip. With ids != nullptr a launch takes the scan path (grid.y =
 // expert, routes collected from ids); otherwise offsets/sorted blocks.

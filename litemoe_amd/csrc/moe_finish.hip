@@ -1,8 +1,8 @@
 // Weighted combine of route outputs (the moe_finish contract):
 //   out[t] = bf16( sum_{j in ascending logical(ids[t,j])*K + j}
 //                  bf16(bf16(y[row(t,j)]) * bf16(scales[t,j])) )   (fp32 sum)
-// Non-owned routes are skipped: nothing of their rows enters the sum (and
-// behind an inverse map, which need not name them, they are never read).
+// Non-owned routes are skipped and, except where the caller says that all of
+// y may be read (kDirect: the library's own scratch), their rows never read.
 // Reference: litemoe/moe_finish.py:7-31 (`_finish`), :34-57 (`finish`).
 #include "internal.h"
 
@@ -12,6 +12,7 @@ namespace {
 constexpr int kMaxK = 8;
 
 // grid (tokens, column blocks); each thread owns kCols consecutive columns.
+// kDirect: rows in route order, every one of them readable.
 template <int kCols, bool kDirect = false>
 __global__ void __launch_bounds__(256)
 finish_kernel(const bf16 *__restrict__ y, const int32_t *__restrict__ ids,
@@ -32,10 +33,10 @@ finish_kernel(const bf16 *__restrict__ y, const int32_t *__restrict__ ids,
   // share the token, so ids, keys and ranks are uniform (scalar registers)
   // and the ordered sum below branches uniformly.
   // kDirect: lane j loads route j's id and scale, and every route row is
-  // requested with them (a row that is not owned is loaded and its values
-  // dropped), so the kernel waits on memory once instead of once per scalar
-  // load and branch (the operator of 700 tokens, hidden 1536, with the norm
-  // behind it: 90.4 -> 88.2 us).
+  // requested with them (the row of an id outside every expert is loaded and
+  // its values dropped), so the kernel waits on memory once instead of once
+  // per scalar load and branch (the operator of 700 tokens, hidden 1536, with
+  // the norm behind it: 90.4 -> 88.2 us).
   u32x4 yv[kDirect ? kMaxK : 1];
   int id_lane = 0;
   float sc_lane = 0.f;
@@ -266,11 +267,11 @@ invert_kernel(const int64_t *__restrict__ order, int64_t n, int32_t *__restrict_
 
 int launch_finish(const bf16 *y, const int32_t *ids, const int32_t *inverse, const float *scales,
                   const int64_t *logical, bf16 *out, int64_t tokens, int64_t hidden, int64_t topk,
-                  int64_t rank, int64_t count, hipStream_t stream) {
+                  int64_t rank, int64_t count, bool y_readable, hipStream_t stream) {
   if (tokens == 0) return LM_OK;
   if (hidden % 8 == 0) {
     const dim3 grid((unsigned)tokens, (unsigned)cdiv(hidden, 256 * 8));
-    auto kernel = inverse ? finish_kernel<8> : finish_kernel<8, true>;
+    auto kernel = y_readable && !inverse ? finish_kernel<8, true> : finish_kernel<8>;
     kernel<<<grid, 256, 0, stream>>>(y, ids, inverse, scales, logical, out, (int)hidden, (int)topk, rank,
                                      count);
   } else {
@@ -303,8 +304,9 @@ extern "C" int lm_moe_finish(const void *y, const int32_t *ids, const int64_t *o
     invert_kernel<<<dim3((unsigned)cdiv(routes, 256)), 256, 0, s>>>(order, routes, inverse);
     LM_CHECK_LAUNCH();
   }
+  // y may hold no more than the owned rows, or rows that another rank still writes.
   return launch_finish((const bf16 *)y, ids, inverse, scales, logical, (bf16 *)out, tokens, hidden,
-                       topk, rank, count, s);
+                       topk, rank, count, /*y_readable=*/false, s);
 }
 
 extern "C" int lm_moe_finish_add_rmsnorm(const void *y, const int32_t *ids, const float *scales,

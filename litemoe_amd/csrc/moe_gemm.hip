@@ -1137,7 +1137,7 @@ int fused_experts(const void *x, const void *w13, const void *w2, const float *t
                       w, packed, stream);
   if (rc) return rc;
   return launch_finish(w.y, topk_ids, nullptr, topk_weights, logical, (bf16 *)out, tokens, hidden,
-                       topk, 0, experts, (hipStream_t)stream);
+                       topk, 0, experts, /*y_readable=*/true, (hipStream_t)stream);
 }
 
 // One thread per 16-byte chunk (tile, k-step, lane) of the fragment layout.
@@ -1329,5 +1329,5 @@ extern "C" int lm_fused_experts_noalloc(const void *x, const void *w13, const vo
                             w.y, w, false, stream);
   if (rr) return rr;
   return launch_finish(w.y, topk_ids, nullptr, topk_weights, logical, (bf16 *)out, tokens, hidden,
-                       topk, 0, experts, (hipStream_t)stream);
+                       topk, 0, experts, /*y_readable=*/true, (hipStream_t)stream);
 }

@@ -166,3 +166,17 @@ def test_single_hip_runtime_in_process():
     import torch  # noqa: F401  (loads torch's HIP runtime)
     _lib.load()
     _lib._check_single_runtime()
+
+
+def test_public_combine_reads_owned_rows_only():
+    """The header says of lm_moe_finish that rows of routes it does not own
+    are never read, so it may not take the kernel that requests every row
+    before it knows the owners: that one runs on the library's own scratch."""
+    csrc = HEADER.parents[1] / "litemoe_amd" / "csrc"
+    finish = (csrc / "moe_finish.hip").read_text()
+    launch = finish[finish.index("int launch_finish("):]
+    assert re.search(r"y_readable && !inverse \? finish_kernel<8, true> : finish_kernel<8>;", launch)
+    public = finish[finish.index('extern "C" int lm_moe_finish('):finish.index('extern "C" int lm_moe_finish_add')]
+    assert "/*y_readable=*/false" in public and "finish_kernel" not in public
+    calls = re.findall(r"launch_finish\((.+?)\);", (csrc / "moe_gemm.hip").read_text(), re.S)
+    assert calls and all(c.startswith("w.y,") and "/*y_readable=*/true" in c for c in calls)

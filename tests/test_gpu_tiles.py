@@ -181,3 +181,41 @@ def test_few_routes_equal_block_path(m, h, i, e, k, hot, packed):
     ids = ids.to(DEV)
     w = experts.pack_expert_weights(w1, w2) if packed else (w1, w2)
     assert torch.equal(experts.moe_routes(x, *w, ids, packed=packed), experts.moe_routes(x, w1, w2, ids, block_rows=16))
+
+
+@torch.inference_mode()
+def test_finish_in_route_order_takes_y_of_the_owned_rows_only():
+    """Routes of other ranks have no row behind y: the first tokens hold the
+    owned routes, and y ends with the last of them."""
+    g = torch.Generator().manual_seed(3)
+    batch, topk, hidden, count, rank = 40, 8, 1536, 8, 1
+    ids = torch.stack([torch.randperm(count, generator=g)[:topk] for _ in range(batch)]).int()
+    ids[:7, ::2] += rank * count
+    owned = (ids.flatten() >= count).nonzero().flatten()
+    y = torch.randn(batch * topk, hidden, generator=g).to(torch.bfloat16)
+    scales = torch.softmax(torch.randn(batch, topk, generator=g), -1)
+    d = [t.to(DEV) for t in (y[:int(owned[-1]) + 1], ids, scales)]
+    out = torch.full((batch, hidden), 7.0, dtype=torch.bfloat16, device=DEV)
+    _lib.call("lm_moe_finish", d[0].data_ptr(), d[1].data_ptr(), None, d[2].data_ptr(), None, out.data_ptr(), batch,
+              hidden, topk, rank, count, None, 0, _lib.stream(out.device))
+    assert torch.equal(out.cpu(), ops.finish(y, ids, scales, rank, count, None))
+
+
+@pytest.mark.parametrize("m,h,i,e,k", [(3, 128, 128, 9, 3), (700, 1536, 128, 16, 8), (300, 2048, 128, 16, 8)])
+@torch.inference_mode()
+def test_fused_experts_combine_drops_ids_of_no_expert(m, h, i, e, k):
+    """The combine that loads every row of the library's scratch: ids outside
+    every expert add nothing, whatever their rows hold."""
+    g = torch.Generator().manual_seed(m)
+    x = torch.randn(m, h, generator=g).to(torch.bfloat16).to(DEV)
+    w1 = (torch.randn(e, 2 * i, h, generator=g) * 0.05).to(torch.bfloat16).to(DEV)
+    w2 = (torch.randn(e, h, i, generator=g) * 0.05).to(torch.bfloat16).to(DEV)
+    ids = torch.stack([torch.randperm(e, generator=g)[:k] for _ in range(m)]).int()
+    ids[::3, 0] = e
+    ids[1::3, -1] = -1
+    scales = torch.softmax(torch.randn(m, k, generator=g), -1)
+    backend = experts.HipFusedExperts()
+    backend.workspace.get(x.device, 1 << 26).fill_(0xFF)  # NaN in every row that is not written
+    out = backend.operation(x, w1, w2, scales.to(DEV), ids.to(DEV), global_num_experts=e)
+    y = experts.moe_routes(x, w1, w2, ids.to(DEV)).cpu()
+    assert torch.equal(out.cpu(), ops.finish(y, ids, scales, 0, e, None))
