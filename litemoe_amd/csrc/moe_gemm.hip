@@ -294,7 +294,12 @@ gate_up_kernel(const bf16 *__restrict__ x, const bf16 *__restrict__ w13,
 // 1280 weight tiles (Granite-3B shape) are in flight at once instead of 768.
 // kFew: at most kFewRoutes routes, found by find_few, the weights requested
 // only by the workgroups of experts that have some (a call of a few tokens
-// leaves most experts out).
+// leaves most experts out). An expert's tiles then spread over all XCDs
+// instead of xcd_tile's one: of the few experts with routes, some share an
+// XCD and some XCDs have none (24 layers of hidden 1024, 32 experts, with
+// combine and norm, us: 1 row 383 -> 348, 3 rows 507 -> 468, 8 rows 580 ->
+// 566, 15 rows 602 -> 607; of hidden 1536, 40 experts: 1 row 502 -> 454, 5
+// rows 794 -> 703, 15 rows 938 -> 907).
 template <int KS, bool kPacked, bool kFew = false>
 __global__ void __launch_bounds__(kThreads, KS <= 12 ? 4 : 2)
 gate_up_scan_kernel(const bf16 *__restrict__ x, const bf16 *__restrict__ w13,
@@ -309,8 +314,8 @@ gate_up_scan_kernel(const bf16 *__restrict__ x, const bf16 *__restrict__ w13,
   __shared__ int wave_count[kWaves];
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int col = lane % 16, grp = lane / 16;
-  int e, tile;
-  xcd_tile(e, tile);
+  int e = blockIdx.y, tile = blockIdx.x;
+  if constexpr (!kFew) xcd_tile(e, tile);
   const int n0 = tile * 16;
   const int kbase = wave * KS * 32 + grp * 8;
   const int64_t rg = (int64_t)e * 2 * inter + n0 + col;
@@ -641,8 +646,8 @@ down_scan_kernel(const bf16 *__restrict__ act, const bf16 *__restrict__ w2,
   __shared__ int last_flag;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int col = lane % 16, grp = lane / 16;
-  int e, tile;
-  xcd_tile(e, tile);
+  int e = blockIdx.y, tile = blockIdx.x;
+  if constexpr (!kFew) xcd_tile(e, tile);
   const int n0 = tile * 16 * NT;
   const int kbase = wave * KS * 32 + grp * 8;
   const int64_t r0 = (int64_t)e * hidden + n0 + col;
@@ -755,9 +760,9 @@ bool ks_ok(int64_t n) {
 
 // Weight tiles are prefetched before the route scan when an empty expert is
 // unlikely (>= 4 routes per expert on average): four layers at hidden 1536, 40
-// experts, us: 24 rows 157.5 against 164 without the prefetch (167 and 170
-// with half of the routes on four experts), 10 rows 158 against 152 (156 and
-// 144 with them).
+// experts, us: 24 rows 154 against 158 without the prefetch (166 and 163 with
+// half of the routes on four experts; 24 layers 925 and 951, 997 and 973), 19
+// rows 156 and 156 (164 and 156), 10 rows 157 against 145 (156 and 132).
 int route_mode(bool scan, int64_t routes, int64_t experts) {
   if (!scan) return kBlocks;
   if (routes >= 4 * experts) return kScanPrefetch;
