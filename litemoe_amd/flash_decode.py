@@ -29,13 +29,23 @@ def default_splits(batch, kv_heads, maximum, target_workgroups=512, min_keys=256
     combine. Measured as the attention block of a decode graph, us per layer,
     against splits for the whole target: 24 rows x 8 heads to 2000 keys 31.3
     (1 split) and 36.9 (3); 10 rows 24.7 (3) and 29.5 (7); 3 rows to 4001 keys
-    21.2 (10) and 23.2 (15); 32 rows to 1500 27.6 (1) and 30.2 (2). Beyond it,
-    the splits bring the workgroups to the target (40 rows to 4000 keys 70.8
-    with 2 splits, 73.5 with 1). A split keeps at least ``min_keys`` keys, and
-    contexts below three times that are not split, since their combine costs
-    more than the shorter stream saves (one row, 512 keys: 16.4 and 17.4)."""
+    21.2 (10) and 23.2 (15); 32 rows to 1500 27.6 (1) and 30.2 (2). Where that
+    is one split and leaves two fifths of the CUs without a workgroup, three
+    take its place if each keeps four times ``min_keys`` keys: they cost equal
+    lengths nothing and serve ragged ones better (17 rows to 4095 keys, 3
+    splits against 1, lengths from three quarters of it up 40.6 and 40.4, from
+    a quarter 37.6 and 39.4, from a tenth 37.0 and 39.0; to 2000 keys 28.7 and
+    27.7). With more rows they cost equal lengths as much (21 rows 43.4 and
+    42.9, from a quarter 40.2 and 40.8) or more (24 rows 50.5 and 45.8; from a
+    quarter 41.6 and 43.3). Beyond half of the target, the splits bring the
+    workgroups to it (40 rows to 4000 keys 70.8 with 2 splits, 73.5 with 1). A
+    split keeps at least ``min_keys`` keys, and contexts below three times
+    that are not split, since their combine costs more than the shorter stream
+    saves (one row, 512 keys: 16.4 and 17.4)."""
     pairs, half = max(1, batch * kv_heads), target_workgroups // 2
     want = half // pairs if pairs <= half else math.ceil(target_workgroups / pairs)
+    if want == 1 and 5 * pairs <= 3 * half and maximum >= 12 * min_keys:
+        want = 3
     longest = maximum // min_keys if maximum >= 3 * min_keys else 1
     return max(1, min(max_splits, want, longest))
 
