@@ -39,6 +39,7 @@ namespace {
 constexpr int kBK = 64;   // K per stage
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, each with its own L2
 constexpr int kRowBytes = kBK * 2;  // 128
+constexpr int kLdsBytes = 160 * 1024;  // per CU
 
 template <int TM, int TN, int WMv, int WNv, int StagesV>
 struct TileCfg {
@@ -163,7 +164,26 @@ expert_gemm_kernel(const bf16 *__restrict__ a_src, const bf16 *__restrict__ w,
   // two stages are two arrays, three one array
   __shared__ __align__(16) char smem[kStages == 2 ? kStageBytes : kStages * kStageBytes];
   __shared__ __align__(16) char smem1[kStages == 2 ? kStageBytes : 16];
-  __shared__ int route_of[kTM];
+  constexpr int kOutCols = kGateUp ? kTN / 2 : kTN, kOB = kOutCols * 2;  // output row bytes
+  constexpr int kHalfRows = (kStages == 2 ? 1 : kStages) * kStageBytes / kOB;  // staged output rows in smem
+  static_assert(kTM * kOB <= kStages * kStageBytes, "output tile fits the LDS stages");
+  // The output rows' routes (all forms but gate_up on sorted act), for the
+  // epilogue only: in the stages behind the staged output tile where there is
+  // room, since the 192 x 128 tile's two workgroups per CU need all 160 KB for
+  // their stages (1200 routes per expert, us: gate_up on route-order act at
+  // hidden 1536, 40 experts, 193 -> 144, down at hidden 384, 32 experts, 29.5
+  // -> 23.6).
+  constexpr bool kRouteList = !(kGateUp && kSortedAct);
+  constexpr int kTileEnd = kTM * kOB, kListBytes = kTM * 4, kSmem1 = kStages == 2 ? kStageBytes : 0;
+  constexpr bool kBehind0 = kTileEnd + kListBytes <= (int)sizeof(smem);
+  constexpr int kUsed1 = kTM > kHalfRows ? (kTM - kHalfRows) * kOB : 0;
+  constexpr bool kBehind1 = !kBehind0 && kUsed1 + kListBytes <= kSmem1;
+  constexpr bool kOwnList = kRouteList && !kBehind0 && !kBehind1;
+  static_assert(!kOwnList || 2 * kStages * kStageBytes > kLdsBytes, "the list takes the second workgroup's room");
+  __shared__ int list_own[kOwnList ? kTM : 1];
+  int *const route_of = kBehind0   ? reinterpret_cast<int *>(smem + kTileEnd)
+                        : kBehind1 ? reinterpret_cast<int *>(smem1 + kUsed1)
+                                   : list_own;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   // Each XCD takes a contiguous range of route blocks with all their column
   // tiles (block_of): a block's gathered A rows are then fetched into one L2,
@@ -175,19 +195,10 @@ expert_gemm_kernel(const bf16 *__restrict__ a_src, const bf16 *__restrict__ w,
   if (!block_of(offsets, experts, kTM, lin, cols, e, r0, r1)) return;
   const int n = r1 - r0;
   const int c0 = tile_x * (kGateUp ? kTN / 2 : kTN);  // first output column
-  // The route list in LDS serves the A row offsets of gate_up and of down on
-  // route-order act, and y's rows in down's epilogue. gate_up on sorted act
-  // reads each row's route directly (no LDS round, no barrier); down on
-  // sorted act fills the list only after its first k step's copies are out
-  // (its rows are the block's own), so the two load round trips overlap.
-  constexpr bool kRouteList = !(kGateUp && kSortedAct), kListFirst = !kSortedAct;
-  auto fill_routes = [&]() {
-    for (int t = threadIdx.x; t < kTM; t += kThreadsT) route_of[t] = sorted[r0 + min(t, n - 1)];
-  };
-  if constexpr (kListFirst) {
-    fill_routes();
-    __syncthreads();
-  }
+  // This thread's entry of the route list, requested ahead of the K loop.
+  static_assert(kTM <= kThreadsT, "a list entry per thread");
+  [[maybe_unused]] int my_route = 0;
+  if constexpr (kRouteList) my_route = sorted[r0 + min((int)threadIdx.x, n - 1)];
 
   // Load instruction i of wave w fills LDS rows 8*(w*L+i) .. +7 of an
   // operand (1 KB, lane l at byte 16*l): row 8*(w*L+i) + l/8, position l%8,
@@ -200,7 +211,7 @@ expert_gemm_kernel(const bf16 *__restrict__ a_src, const bf16 *__restrict__ w,
     if constexpr (!kGateUp && kSortedAct) {
       oa[i] = (r0 + min(t, n - 1)) * K + chunk * 8;
     } else {
-      const int route = kListFirst ? route_of[t] : sorted[r0 + min(t, n - 1)];
+      const int route = sorted[r0 + min(t, n - 1)];
       oa[i] = (kGateUp ? route / topk : route) * K + chunk * 8;
     }
   }
@@ -289,8 +300,6 @@ expert_gemm_kernel(const bf16 *__restrict__ a_src, const bf16 *__restrict__ w,
     };
     issue_a(0, smem);
     issue_b(0, smem);
-    // published by the first barrier below; read only in the epilogue
-    if constexpr (kRouteList && !kListFirst) fill_routes();
     for (int kt = 0; kt < nk; kt += 2) {
       lds_copy_wait();
       __syncthreads();
@@ -327,7 +336,6 @@ expert_gemm_kernel(const bf16 *__restrict__ a_src, const bf16 *__restrict__ w,
 #pragma unroll
     for (int s = 0; s < kStages - 1; ++s)
       if (s < nk) issue(s, smem + s * kStageBytes);
-    if constexpr (kRouteList && !kListFirst) fill_routes();
     int cur = 0, nxt = (kStages - 1) * kStageBytes;
     for (int kt = 0; kt < nk; ++kt) {
       if (kt + 1 < nk) vm_wait<kL>(); else vm_wait<0>();
@@ -349,15 +357,14 @@ expert_gemm_kernel(const bf16 *__restrict__ a_src, const bf16 *__restrict__ w,
   // covers whole output rows (512 or 256 bytes each) instead of 32-byte
   // pieces of 16 rows. Staged row r's 16-byte chunk c sits at c ^ (r & kSw):
   // the 16 rows of one fragment store fall on different bank groups.
-  constexpr int kOutCols = kGateUp ? kTN / 2 : kTN, kOB = kOutCols * 2;  // output row bytes
   constexpr int kChunks = kOB / 16, kSw = (kChunks < 16 ? kChunks : 16) - 1;
-  constexpr int kHalfRows = (kStages == 2 ? 1 : kStages) * kStageBytes / kOB;  // rows held by smem
-  static_assert(kTM * kOB <= kStages * kStageBytes, "output tile fits the LDS stages");
   auto staged = [&](int row) -> char * {
     if constexpr (kTM <= kHalfRows) return smem + row * kOB;
     else return row < kHalfRows ? smem + row * kOB : smem1 + (row - kHalfRows) * kOB;
   };
   __syncthreads();  // every wave has finished reading the stages
+  if constexpr (kRouteList)
+    if (threadIdx.x < kTM) route_of[threadIdx.x] = my_route;
 #pragma unroll
   for (int rb = 0; rb < kRB; ++rb) {
     const int row = wr * kWaveRows + rb * 16 + fr;

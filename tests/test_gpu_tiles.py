@@ -219,3 +219,23 @@ def test_fused_experts_combine_drops_ids_of_no_expert(m, h, i, e, k):
     out = backend.operation(x, w1, w2, scales.to(DEV), ids.to(DEV), global_num_experts=e)
     y = experts.moe_routes(x, w1, w2, ids.to(DEV)).cpu()
     assert torch.equal(out.cpu(), ops.finish(y, ids, scales, 0, e, None))
+
+
+@pytest.mark.parametrize("m,h,e", [
+    (300, 384, 32), (600, 384, 32), (1300, 256, 96), (900, 384, 7), (2049, 256, 8), (1200, 1536, 8), (4100, 384, 16)])
+@torch.inference_mode()
+def test_expert_stages_equal_fused_routes(m, h, e):
+    """lm_moe_gate_up and lm_moe_down on aligned routes (act in route order, the
+    route list behind the staged tile or its own) against lm_moe_routes (act in
+    sorted order), bit for bit, ids of no expert among them."""
+    g = torch.Generator().manual_seed(m)
+    x = torch.randn(m, h, generator=g).to(torch.bfloat16).to(DEV)
+    w1 = (torch.randn(e, 256, h, generator=g) * 0.05).to(torch.bfloat16).to(DEV)
+    w2 = (torch.randn(e, h, 128, generator=g) * 0.05).to(torch.bfloat16).to(DEV)
+    ids = torch.stack([torch.randperm(e + 1, generator=g)[:7] for _ in range(m)]).int().to(DEV)
+    offsets, order, _ = experts.moe_align(ids, e)
+    act = experts.gate_up(x, w1, offsets, order, 7)
+    y = experts.down(act, w2, offsets, order)
+    expected = torch.zeros_like(y)
+    experts.moe_routes(x, w1, w2, ids, y=expected)
+    assert torch.equal(y, expected)
