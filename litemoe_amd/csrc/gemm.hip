@@ -32,10 +32,23 @@
 // 103.0-103.3 ms, A/B on one box); otherwise each lane stores its four
 // columns as one 8-byte word (or 2-byte stores for odd widths).
 //
-// Workgroups are dealt to the 8 XCDs round-robin in launch order; they are
-// remapped so each XCD takes a contiguous range of row tiles with all their
-// column tiles: a row tile's A rows are fetched into one L2 and reused there
-// by every column tile.
+// Workgroups are dealt to the 8 XCDs round-robin in launch order, and the
+// tiles (TileOrder) so that each XCD takes a contiguous range of row tiles
+// with all their column tiles: a row tile's A rows are fetched into one L2 and
+// reused there by every column tile. Where whole row tiles would leave the
+// fullest CU more tiles than eighths of all tiles do (nine row tiles keep five
+// of the eight XCDs busy), each XCD takes an eighth: by row, or, where W is
+// twice A or A fits an L2, by column, since the operand that is not dealt is
+// fetched into every L2. lm_linear with cold weights, us, whole row tiles /
+// eighths by row / by column (* taken):
+//   513 x 1536 x 1536  11.7   9.2    8.1*      4955 x 2786 x 1536  101   57*  57
+//   563 x 6300 x 1024  30.8  18.8   12.7*     13000 x 2560 x 1536  109   81*
+//  1911 x 4480 x 2048  63.2  42.1   42.8*     25000 x 2560 x 1536  186  154*
+//   734 x 5271 x 1536  42.6  31.0   23.7*      3301 x 5012 x 2048   89   74*  80
+//  1317 x 1852 x 1536  14.7* 16.5   16.4       5854 x 6112 x 4096  269*      320
+// Fewer row tiles than XCDs stay in launch order: an XCD's column tiles then
+// lie eight apart (276 x 13578 x 512 15.6 us, by column 18.3; 741 x 11598 x
+// 2048 54.9 and 61.2).
 //
 // Reference: the packed QKV and output projections of litemoe/model.py:47-49
 // and :60 (F.linear over the packed prefill rows), and the LM head :127.
@@ -48,6 +61,8 @@ namespace {
 
 constexpr int kBK = 64;
 constexpr int kXcds = 8;
+constexpr int64_t kCus = 256, kL2Bytes = 4 << 20;  // an XCD's L2
+enum TileOrder : int { kPlain, kByRow, kByColumn };
 constexpr int kRowBytes = kBK * 2;  // 128
 
 __device__ __forceinline__ int frag_offset(int row, int chunk) {
@@ -82,7 +97,7 @@ template <int kTM, int kTN, int kWM, int kWN, int kStages, int kStore, bool kRop
 __global__ void __launch_bounds__(64 * kWM * kWN)
 gemm_kernel(const bf16 *__restrict__ a, int64_t lda, const bf16 *__restrict__ w, int64_t ldw,
             bf16 *__restrict__ out, int64_t ldo, int M, int N, int K, int tiles_m, int tiles_n,
-            int xcd_remap, RopeKV rk) {
+            int order, int per_xcd, RopeKV rk) {
   constexpr int kWaves = kWM * kWN;
   constexpr int kWaveRows = kTM / kWM, kWaveCols = kTN / kWN;
   constexpr int kRB = kWaveRows / 16, kCB = kWaveCols / 16;
@@ -109,13 +124,14 @@ gemm_kernel(const bf16 *__restrict__ a, int64_t lda, const bf16 *__restrict__ w,
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int lin = blockIdx.x;
   int tile_m = lin / tiles_n, tile_n = lin % tiles_n;
-  if (xcd_remap) {  // grid = tiles_n * (tiles_m rounded up to a multiple of 8)
-    const int per_xcd = (int)(gridDim.x / kXcds) / tiles_n;  // row tiles per XCD
-    const int j = lin / kXcds;
-    tile_m = (lin % kXcds) * per_xcd + j / tiles_n;
-    tile_n = j % tiles_n;
+  if (order != kPlain) {
+    const int tile = lin % kXcds * per_xcd + lin / kXcds;
+    const int run = order == kByColumn ? tiles_m : tiles_n;
+    const int outer = tile / run, inner = tile - outer * run;
+    tile_m = order == kByColumn ? inner : outer;
+    tile_n = order == kByColumn ? outer : inner;
   }
-  if (tile_m >= tiles_m) return;
+  if (tile_m >= tiles_m || tile_n >= tiles_n) return;
   const int m0 = tile_m * kTM, n0 = tile_n * kTN;
 
   // Copy instruction i of wave w fills LDS rows 8*(w*L+i) .. +7 of an
@@ -421,17 +437,20 @@ template <int TM, int TN, int WM, int WN, int Stages, bool kRope>
 int launch_gemm_cfg(const bf16 *a, int64_t lda, const bf16 *w, int64_t ldw, bf16 *out, int64_t ldo,
                     int64_t M, int64_t N, int64_t K, hipStream_t stream, const RopeKV &rope) {
   const int64_t tiles_m = cdiv(M, TM), tiles_n = cdiv(N, TN);
-  // With fewer row tiles than XCDs the remap would put every tile on a few
-  // XCDs; the plain order spreads the column tiles instead.
-  const bool remap = tiles_m >= kXcds;
-  const int64_t blocks = (remap ? align_up(tiles_m, kXcds) : tiles_m) * tiles_n;
+  // (tiles of the fullest CU, dealt by whole row tiles and by eighths)
+  const int64_t rows = align_up(tiles_m, kXcds) * tiles_n, even = align_up(tiles_m * tiles_n, kXcds);
+  const bool eighths = tiles_m >= kXcds && cdiv(even, kCus) < cdiv(rows, kCus);
+  const bool by_column = eighths && (2 * M <= N || (M < N && 2 * M * K <= kL2Bytes));
+  const int order = tiles_m < kXcds ? kPlain : by_column ? kByColumn : kByRow;
+  const int64_t blocks = order == kPlain ? tiles_m * tiles_n : eighths ? even : rows;
   const bool vec = N % 4 == 0 && ldo % 4 == 0 && ((uintptr_t)out & 7) == 0;
   const bool vec16 = N % 8 == 0 && ldo % 8 == 0 && ((uintptr_t)out & 15) == 0;
   const dim3 grid((unsigned)blocks);
   auto go = [&](auto store_c) {
     gemm_kernel<TM, TN, WM, WN, Stages, decltype(store_c)::value, kRope>
         <<<grid, 64 * WM * WN, 0, stream>>>(a, lda, w, ldw, out, ldo, (int)M, (int)N, (int)K,
-                                            (int)tiles_m, (int)tiles_n, (int)remap, rope);
+                                            (int)tiles_m, (int)tiles_n, order,
+                                            (int)(blocks / kXcds), rope);
   };
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;

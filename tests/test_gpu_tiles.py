@@ -239,3 +239,17 @@ def test_expert_stages_equal_fused_routes(m, h, e):
     expected = torch.zeros_like(y)
     experts.moe_routes(x, w1, w2, ids, y=expected)
     assert torch.equal(y, expected)
+
+
+@pytest.mark.parametrize("rows,n,k", [
+    (513, 1536, 64), (563, 6300, 128), (734, 5271, 64),      # each XCD an eighth of the tiles, by column
+    (4955, 2786, 64), (2904, 4523, 1024),                    # by row
+    (1317, 1852, 64), (575, 6400, 64)])                      # whole row tiles, fewer row tiles than XCDs
+@torch.inference_mode()
+def test_linear_dense_tile_orders(rows, n, k):
+    test_linear_dense_tiles_match_fp32_product(rows, n, k)
+
+
+@torch.inference_mode()
+def test_linear_rope_kv_tiles_dealt_by_eighths():
+    projections.test_linear_rope_kv_equals_projection_then_rope_kv_write(6400, 24, 8, 64, 13, 512, 512, True)
