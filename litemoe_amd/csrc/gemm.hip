@@ -498,8 +498,20 @@ int launch_gemm_tiled(const bf16 *a, int64_t lda, const bf16 *w, int64_t ldw, bf
     // (a rope wave holds one head: 64 columns)
     if (tiles(64, 64) <= 256) return launch_gemm_cfg<64, 64, kRope ? 4 : 2, kRope ? 1 : 2, 3, kRope>;
     if (tiles(128, 64) <= 256) return launch_gemm_cfg<128, 64, 4, 1, 3, kRope>;
+    // Up to 64 and 128 rows one row tile reads the weights once, whatever the
+    // grid (before: 64 x 128 to 512 tiles, 128 x 128, 192 x 128 and 256 x 256
+    // beyond). Where 64 x 128 tiles are more than one to a CU, 64 x 256 ones in
+    // three stages have more weight bytes in flight, to four fifths of
+    // a round of themselves. Cold weights, us, before / now: 48 x 49155 x 1536
+    // 37.2 / 34.1, 64 x 49155 x 1024 27.3 / 24.7, 32 x 66000 x 1536 65.6 / 47.7,
+    // 64 x 152064 x 1024 94.9 / 63.8, 100 x 128256 x 1536 103.8 / 93.3.
+    if constexpr (!kRope) {
+      if (M <= 64 && tiles(64, 128) > 256 && tiles(64, 256) <= 208)
+        return launch_gemm_cfg<64, 256, 2, 4, 3, false>;
+      if (M <= 64) return launch_gemm_cfg<64, 128, 2, 2, 3, false>;
+    }
     if (tiles(64, 128) <= 512) return launch_gemm_cfg<64, 128, 2, 2, 3, kRope>;
-    if (tiles(128, 128) <= 512) return launch_gemm_cfg<128, 128, 4, 2, 2, kRope>;
+    if (M <= 128 || tiles(128, 128) <= 512) return launch_gemm_cfg<128, 128, 4, 2, 2, kRope>;
     // Beyond one round, 256 x 256 tiles take less time per output unless their
     // last round is mostly empty: below three quarters of the slots that their
     // rounds have, 192 x 128 (two per CU) are faster (7584 x 2560 x 1536 64.4

@@ -253,3 +253,12 @@ def test_linear_dense_tile_orders(rows, n, k):
 @torch.inference_mode()
 def test_linear_rope_kv_tiles_dealt_by_eighths():
     projections.test_linear_rope_kv_equals_projection_then_rope_kv_write(6400, 24, 8, 64, 13, 512, 512, True)
+
+
+@pytest.mark.parametrize("rows,n,k", [
+    (17, 32769, 64), (64, 40003, 192), (33, 53248, 128),     # 64 x 256, three stages
+    (64, 53249, 64), (40, 66001, 128),                       # 64 x 128 past them
+    (65, 66000, 64), (128, 70001, 128)])                     # 128 x 128, any number of column tiles
+@torch.inference_mode()
+def test_linear_dense_one_row_tile(rows, n, k):
+    test_linear_dense_tiles_match_fp32_product(rows, n, k)
