@@ -433,16 +433,23 @@ gemm_kernel(const bf16 *__restrict__ a, int64_t lda, const bf16 *__restrict__ w,
   }
 }
 
+// Whether the tiles are dealt by eighths: tiles of the fullest CU, dealt so and
+// by whole row tiles.
+bool by_eighths(int64_t tiles_m, int64_t tiles_n) {
+  return tiles_m >= kXcds &&
+         cdiv(align_up(tiles_m * tiles_n, kXcds), kCus) < cdiv(align_up(tiles_m, kXcds) * tiles_n, kCus);
+}
+
 template <int TM, int TN, int WM, int WN, int Stages, bool kRope>
 int launch_gemm_cfg(const bf16 *a, int64_t lda, const bf16 *w, int64_t ldw, bf16 *out, int64_t ldo,
                     int64_t M, int64_t N, int64_t K, hipStream_t stream, const RopeKV &rope) {
   const int64_t tiles_m = cdiv(M, TM), tiles_n = cdiv(N, TN);
-  // (tiles of the fullest CU, dealt by whole row tiles and by eighths)
-  const int64_t rows = align_up(tiles_m, kXcds) * tiles_n, even = align_up(tiles_m * tiles_n, kXcds);
-  const bool eighths = tiles_m >= kXcds && cdiv(even, kCus) < cdiv(rows, kCus);
+  const bool eighths = by_eighths(tiles_m, tiles_n);
   const bool by_column = eighths && (2 * M <= N || (M < N && 2 * M * K <= kL2Bytes));
   const int order = tiles_m < kXcds ? kPlain : by_column ? kByColumn : kByRow;
-  const int64_t blocks = order == kPlain ? tiles_m * tiles_n : eighths ? even : rows;
+  const int64_t blocks = order == kPlain ? tiles_m * tiles_n
+                         : eighths     ? align_up(tiles_m * tiles_n, kXcds)
+                                       : align_up(tiles_m, kXcds) * tiles_n;
   const bool vec = N % 4 == 0 && ldo % 4 == 0 && ((uintptr_t)out & 7) == 0;
   const bool vec16 = N % 8 == 0 && ldo % 8 == 0 && ((uintptr_t)out & 15) == 0;
   const dim3 grid((unsigned)blocks);
@@ -510,6 +517,16 @@ int launch_gemm_tiled(const bf16 *a, int64_t lda, const bf16 *w, int64_t ldw, bf
         return launch_gemm_cfg<64, 256, 2, 4, 3, false>;
       if (M <= 64) return launch_gemm_cfg<64, 128, 2, 2, 3, false>;
     }
+    // Where W is the larger operand, 128 x 64 tiles (two per CU as well) read it
+    // half as often as 64 x 128 ones, unless those are dealt by eighths or W is
+    // read twice. Cold weights, us, 64 x 128 / 128 x 64: 89 x 29517 x 4096
+    // 75.6 / 61.9, 354 x 7231 x 4096 63.8 / 43.5, 506 x 4961 x 1024 21.2 / 17.0, 624
+    // x 4076 x 1536 27.5 / 16.4; by eighths 669 x 4212 x 1536 16.2 / 18.9, four row
+    // tiles 198 x 8605 x 1536 18.9 / 21.4, a few tiles past a round 91 x 21461 x
+    // 1024 16.8 / 19.4.
+    const bool narrow = M <= 128 ? tiles(128, 64) > 340 : M > 256 && N >= 3 * M && tiles(64, 128) > 256;
+    if (!kRope && narrow && tiles(128, 64) <= 512 && !by_eighths(cdiv(M, 64), cdiv(N, 128)))
+      return launch_gemm_cfg<128, 64, 4, 1, 3, kRope>;
     if (tiles(64, 128) <= 512) return launch_gemm_cfg<64, 128, 2, 2, 3, kRope>;
     if (M <= 128 || tiles(128, 128) <= 512) return launch_gemm_cfg<128, 128, 4, 2, 2, kRope>;
     // Beyond one round, 256 x 256 tiles take less time per output unless their

@@ -262,3 +262,11 @@ def test_linear_rope_kv_tiles_dealt_by_eighths():
 @torch.inference_mode()
 def test_linear_dense_one_row_tile(rows, n, k):
     test_linear_dense_tiles_match_fp32_product(rows, n, k)
+
+
+@pytest.mark.parametrize("rows,n,k", [
+    (65, 21761, 64), (100, 24001, 192), (128, 32768, 64), (128, 32769, 128),  # 341 to 512 tiles of 128 x 64, and past them
+    (257, 6700, 64), (506, 4961, 192), (624, 4076, 64)])
+@torch.inference_mode()
+def test_linear_dense_narrow_tiles_of_wide_outputs(rows, n, k):
+    test_linear_dense_tiles_match_fp32_product(rows, n, k)
