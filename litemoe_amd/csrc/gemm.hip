@@ -534,8 +534,12 @@ int launch_gemm_tiled(const bf16 *a, int64_t lda, const bf16 *w, int64_t ldw, bf
     // rounds have, 192 x 128 (two per CU) are faster (7584 x 2560 x 1536 64.4
     // against 70.9 us at 0.59, 10000 x 2560 78.5 against 77.7 at 0.78; 20000 x
     // 1024 x 1024 42.9 against 53.2 at 0.62).
-    const int64_t large = tiles(256, 256);
-    if (tiles(192, 128) <= 512 || 4 * large < 3 * align_up(large, 256))
+    // One of them that pads the rows to four thirds of the other's is out: 237 x
+    // 44635 x 1024, cold weights, 49.3 us with 256 rows, 63.7 with 384; 300 x
+    // 49155 x 1536 86.6 with 384, 99.3 with 512.
+    const int64_t large = tiles(256, 256), rows192 = align_up(M, 192), rows256 = align_up(M, 256);
+    if (4 * rows256 <= 3 * rows192) return launch_gemm_cfg<256, 256, 4, 4, 2, kRope>;
+    if (4 * rows192 <= 3 * rows256 || tiles(192, 128) <= 512 || 4 * large < 3 * align_up(large, 256))
       return launch_gemm_cfg<192, 128, 4, 2, 2, kRope>;
     return launch_gemm_cfg<256, 256, 4, 4, 2, kRope>;
   };

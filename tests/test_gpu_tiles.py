@@ -270,3 +270,11 @@ def test_linear_dense_one_row_tile(rows, n, k):
 @torch.inference_mode()
 def test_linear_dense_narrow_tiles_of_wide_outputs(rows, n, k):
     test_linear_dense_tiles_match_fp32_product(rows, n, k)
+
+
+@pytest.mark.parametrize("rows,n,k", [
+    (193, 35001, 64), (256, 66000, 64),                      # 256 rows where 192 would pad to 384
+    (300, 60001, 64), (520, 34000, 128)])                    # and 192 where 256 would pad by a third
+@torch.inference_mode()
+def test_linear_dense_tile_height_by_padding(rows, n, k):
+    test_linear_dense_tiles_match_fp32_product(rows, n, k)
