@@ -163,7 +163,7 @@ class _Cache:
 @pytest.mark.parametrize("rows,hq,hkv,k,batch,cap,table,masked", [
     (5000, 24, 8, 1536, 6, 1024, 1024, False),   # cfg 3/4 layer shape, 256 x 256 tiles
     (3001, 16, 8, 1024, 4, 1024, 900, True),     # cfg 2 shape; positions past the table
-    (700, 24, 8, 1536, 3, 512, 512, True),       # 128 x 128 tiles
+    (700, 24, 8, 1536, 3, 512, 512, True),       # 128 x 64 tiles
     (37, 8, 4, 512, 2, 64, 64, False), (1, 24, 8, 1536, 1, 16, 16, False)])
 @torch.inference_mode()
 def test_linear_rope_kv_equals_projection_then_rope_kv_write(rows, hq, hkv, k, batch, cap, table, masked):

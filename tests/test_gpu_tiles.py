@@ -17,11 +17,14 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("rows,n,k", [
     (1, 64, 64), (16, 4099, 192), (3, 1000, 1536),                     # 16 x 64, 1 to 24 K steps
     (17, 4099, 64), (129, 1000, 128), (256, 4096, 192),                # 64 x 64 (256 tiles)
-    (257, 4096, 64), (300, 8190, 256),                                 # 128 x 64, then 64 x 128
-    (511, 8192, 64), (512, 8192, 192),                                 # 64 x 128 (512 tiles)
+    (257, 4096, 64), (300, 8190, 256),                                 # 128 x 64
+    (511, 8192, 64), (512, 8192, 192),                                 # 128 x 64 (512 tiles)
+    (1500, 2563, 64), (1400, 2820, 192), (64, 17001, 128),             # 64 x 128
     (513, 8200, 128), (1000, 8190, 64),                                # 128 x 128
     (1600, 5632, 128), (1537, 7000, 64),                               # 192 x 128
-    (3000, 5700, 192), (2100, 16001, 64)])                             # 256 x 256
+    (3000, 5700, 192), (2100, 16001, 64),                              # 192 x 128, two rounds and more
+    (3900, 4095, 192), (3841, 4092, 64), (3900, 4088, 128),            # 256 x 256: 2-, 8- and 16-byte stores
+    (200, 49155, 64)])                                                 # one row tile of it
 @torch.inference_mode()
 def test_linear_dense_tiles_match_fp32_product(rows, n, k):
     """Within one bf16 ulp of the fp32 product (1e-3 where a sum cancels), as
