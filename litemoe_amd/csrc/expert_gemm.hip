@@ -417,32 +417,29 @@ bool expert_gemm_ok(int64_t routes, int64_t hidden, int64_t inter, int64_t exper
 
 namespace {
 
-template <class T>
-int launch_tile(bool gate_up, const bf16 *a, const bf16 *w, const int32_t *offsets,
+template <bool kGateUp, class T>
+int launch_tile(const bf16 *a, const bf16 *w, const int32_t *offsets,
                 const int32_t *sorted, int64_t routes, int64_t topk, int64_t K, int64_t out_cols,
                 int64_t inter, int64_t experts, bf16 *out, bool packed, bool sorted_act,
                 hipStream_t stream) {
   const int64_t blocks = align_up(cdiv(routes, T::M) + experts, kXcds);
   if (blocks > 65535) return LM_EUNSUPPORTED;
-  const int64_t cols = gate_up ? 2 * inter : out_cols;
+  const int64_t cols = kGateUp ? 2 * inter : out_cols;
   const dim3 grid((unsigned)(cols / T::N), (unsigned)blocks);
   const int threads = 64 * T::WM * T::WN;
-  auto go = [&](auto gate_c, auto packed_c, auto sorted_c) {
-    expert_gemm_kernel<decltype(gate_c)::value, T::M, T::N, T::WM, T::WN, T::Stages,
-                       decltype(packed_c)::value, decltype(sorted_c)::value>
+  auto go = [&](auto packed_c, auto sorted_c) {
+    expert_gemm_kernel<kGateUp, T::M, T::N, T::WM, T::WN, T::Stages, decltype(packed_c)::value,
+                       decltype(sorted_c)::value>
         <<<grid, threads, 0, stream>>>(a, w, offsets, sorted, (int)topk, (int)K, (int)out_cols,
                                        (int)inter, (int)experts, out);
   };
   using Y = std::true_type;
   using F = std::false_type;
-  auto by_layout = [&](auto gate_c) {
-    if (packed) {
-      if (sorted_act) go(gate_c, Y{}, Y{}); else go(gate_c, Y{}, F{});
-    } else {
-      if (sorted_act) go(gate_c, F{}, Y{}); else go(gate_c, F{}, F{});
-    }
-  };
-  if (gate_up) by_layout(Y{}); else by_layout(F{});
+  if (packed) {
+    if (sorted_act) go(Y{}, Y{}); else go(Y{}, F{});
+  } else {
+    if (sorted_act) go(F{}, Y{}); else go(F{}, F{});
+  }
   LM_CHECK_LAUNCH();
   return LM_OK;
 }
@@ -453,10 +450,10 @@ int launch_expert_gemm_gate_up(const bf16 *x, const bf16 *w13, const int32_t *of
                                const int32_t *sorted, int64_t routes, int64_t topk, int64_t hidden,
                                int64_t inter, int64_t experts, bf16 *act, bool packed,
                                bool sorted_act, hipStream_t stream) {
-  auto launch = routes < kLowBelow * experts        ? launch_tile<GateLow>
-                : routes < kGateHighFrom * experts ? launch_tile<GateMid>
-                                                   : launch_tile<GateHigh>;
-  return launch(true, x, w13, offsets, sorted, routes, topk, hidden, inter, inter, experts, act,
+  auto launch = routes < kLowBelow * experts       ? launch_tile<true, GateLow>
+                : routes < kGateHighFrom * experts ? launch_tile<true, GateMid>
+                                                   : launch_tile<true, GateHigh>;
+  return launch(x, w13, offsets, sorted, routes, topk, hidden, inter, inter, experts, act,
                 packed, sorted_act, stream);
 }
 
@@ -465,11 +462,11 @@ int launch_expert_gemm_down(const bf16 *act, const bf16 *w2, const int32_t *offs
                             int64_t experts, bf16 *y, bool packed, bool sorted_act,
                             hipStream_t stream) {
   const bool wide = hidden % DownMid::N == 0;
-  auto launch = routes < kLowBelow * experts ? launch_tile<DownLow>
-                : !wide                      ? launch_tile<DownMidNarrow>
-                : routes < kDownHighFrom * experts ? launch_tile<DownMid>
-                                                   : launch_tile<DownHigh>;
-  return launch(false, act, w2, offsets, sorted, routes, 1, inter, hidden, inter, experts, y, packed,
+  auto launch = routes < kLowBelow * experts       ? launch_tile<false, DownLow>
+                : !wide                            ? launch_tile<false, DownMidNarrow>
+                : routes < kDownHighFrom * experts ? launch_tile<false, DownMid>
+                                                   : launch_tile<false, DownHigh>;
+  return launch(act, w2, offsets, sorted, routes, 1, inter, hidden, inter, experts, y, packed,
                 sorted_act, stream);
 }
 

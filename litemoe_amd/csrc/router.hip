@@ -618,10 +618,9 @@ __device__ __forceinline__ void batch_norm_row(bf16 *__restrict__ x, float alpha
   }
 }
 
-// Occupancy target: four waves per SIMD up to hidden 1536 and 48 experts;
-// the 49-64 expert tiles need more registers (three waves), wider rows two.
+// Two waves per SIMD (hidden 2048 to 4096).
 template <int NVL, int NT, bool kNorm, bool kAdd>
-__global__ void __launch_bounds__(kBatchThreads, NVL <= 3 ? (NT <= 3 ? 4 : 3) : 2)
+__global__ void __launch_bounds__(kBatchThreads, 2)
 batched_router_kernel(bf16 *__restrict__ x, const bf16 *__restrict__ a, float alpha,
                       const bf16 *__restrict__ nw, float eps, bf16 *__restrict__ z,
                       const bf16 *__restrict__ wr, int experts, int topk, int renormalize,
@@ -706,26 +705,26 @@ batched_router_kernel(bf16 *__restrict__ x, const bf16 *__restrict__ a, float al
                       tw + (row0 + r) * topk, tid + (row0 + r) * topk);
 }
 
-// The same three phases as a persistent kernel: 256 workgroups of sixteen
-// waves, each over every 256th block of 16 tokens, a token per wave. Wave w
-// holds the K quarter w % 4 of gate tile w / 4 as MFMA B operands for the
-// whole launch, so no block reads the gate weights again;
-// a block's z rows reach the matrix cores through LDS (rows padded by 16
-// bytes: a fragment's 16 rows fall on 16 bank groups) instead of being read
-// back from L2; and the next block's row is in flight from the moment the norm
-// has taken this block's, so HBM streams under the logits and the selection
-// instead of alternating with them. The last tokens % 16 are routed in the
-// per-token kernels' order, one per workgroup, by those whose next block they
-// would be, so there is no tail launch (all of them on one workgroup held the
-// launch back: 1039 tokens of hidden 1536 19.3 -> 11.9 us, 8191 tokens 35.1 ->
-// 29.4, 1039 of hidden 1024 13.9 -> 8.7; 46,990 121.0 -> 120.6); the blocks'
-// x, z and logits are bitwise batched_router_kernel's. The stream bounds it: 577 MB at 46,990
-// tokens of hidden 1536, 40 experts, in 121 us (4.8 TB/s; a large copy
-// reaches 4.9) against 162 us for batched_router_kernel and its tail launch;
-// 2000 tokens 35 -> 13 us; hidden 1024, 32 experts, 46,990 tokens 107 -> 79
-// us. Eight waves of two tokens, each holding its quarter of all gate tiles
-// (two waves per SIMD to hide latency with): 166 us. From hidden 2048 the
-// weights no longer fit beside the rows, and batched_router_kernel stays.
+// The same three phases as a persistent kernel, to hidden 1536: 256 workgroups
+// of sixteen waves, each over every 256th block of 16 tokens, a token per wave.
+// Wave w holds the K quarter w % 4 of gate tile w / 4 as MFMA B operands for
+// the whole launch, so no block reads the gate weights again; a block's z rows
+// reach the matrix cores through LDS (rows padded by 16 bytes: a fragment's 16
+// rows fall on 16 bank groups) instead of being read back from L2; and the next
+// block's row is in flight from the moment the norm has taken this block's, so
+// HBM streams under the logits and the selection instead of alternating with
+// them. The last tokens % 16 are routed in the per-token kernels' order, one
+// per workgroup, by those whose next block they would be, so there is no tail
+// launch (all of them on one workgroup held the launch back: 1039 tokens of
+// hidden 1536 19.3 -> 11.9 us, 8191 tokens 35.1 -> 29.4, 1039 of hidden 1024
+// 13.9 -> 8.7; 46,990 121.0 -> 120.6). The blocks' logits are summed as
+// batched_router_kernel sums them. The stream bounds it: 577 MB at 46,990
+// tokens of hidden 1536, 40 experts, in 121 us (4.8 TB/s; a large copy reaches
+// 4.9) against 162 us for batched_router_kernel and its tail launch; 2000
+// tokens 35 -> 13 us; hidden 1024, 32 experts, 46,990 tokens 107 -> 79 us.
+// Eight waves of two tokens, each holding its quarter of all gate tiles (two
+// waves per SIMD to hide latency with): 166 us. From hidden 2048 the weights no
+// longer fit beside the rows, and batched_router_kernel stays.
 constexpr int kPersistWaves = 16, kPersistThreads = kPersistWaves * kWave, kPersistRows = 16;
 constexpr int64_t kPersistGrid = 256;
 
@@ -862,10 +861,10 @@ persistent_router_kernel(bf16 *__restrict__ x, const bf16 *__restrict__ a, float
                       tid + tail_row * topk);
 }
 
-// Routes every token with persistent_router_kernel, or the first
-// tokens - tokens % kBatchRows tokens with
-// batched_router_kernel when the shape allows it; returns how many it routed
-// (0: none, the per-token kernels route them all).
+// Routes every token with persistent_router_kernel, or the first tokens -
+// tokens % kBatchRows tokens with batched_router_kernel when the shape allows
+// it; returns how many it routed (0: none, the per-token kernels route them
+// all).
 template <bool kNorm, bool kAdd>
 int64_t launch_batched_router(int64_t tokens, int64_t hidden, bf16 *x, const bf16 *a,
                               float alpha, const bf16 *nw, float eps, bf16 *z, const bf16 *wr,
@@ -874,8 +873,8 @@ int64_t launch_batched_router(int64_t tokens, int64_t hidden, bf16 *x, const bf1
   const int nv = fast_nv(hidden);
   if (tokens < kBatchRouterMinTokens || !nv || experts > kWave || experts <= 16) return 0;
 #define LM_PERSIST_ROUTER(NVL, NT)                                                               \
-  if (nv == NVL && (experts + 15) / 16 == NT) {                   \
-    const dim3 pgrid((unsigned)std::min(tokens / kPersistRows + tokens % kPersistRows, kPersistGrid));     \
+  if (nv == NVL && (experts + 15) / 16 == NT) {                                                  \
+    const dim3 pgrid((unsigned)std::min(tokens / kPersistRows + tokens % kPersistRows, kPersistGrid)); \
     persistent_router_kernel<NVL, NT, kNorm, kAdd><<<pgrid, kPersistThreads, 0, s>>>(            \
         x, a, alpha, nw, eps, z, wr, tokens, experts, topk, renormalize, logits_out, tw, tid);   \
     return tokens;                                                                               \
@@ -894,8 +893,7 @@ int64_t launch_batched_router(int64_t tokens, int64_t hidden, bf16 *x, const bf1
     return rows;                                                                                \
   }
 #define LM_BATCH_ROUTER_NT(NVL) LM_BATCH_ROUTER(NVL, 2) LM_BATCH_ROUTER(NVL, 3) LM_BATCH_ROUTER(NVL, 4)
-  LM_BATCH_ROUTER_NT(1) LM_BATCH_ROUTER_NT(2) LM_BATCH_ROUTER_NT(3) LM_BATCH_ROUTER_NT(4)
-  LM_BATCH_ROUTER_NT(6) LM_BATCH_ROUTER_NT(8)
+  LM_BATCH_ROUTER_NT(4) LM_BATCH_ROUTER_NT(6) LM_BATCH_ROUTER_NT(8)
 #undef LM_BATCH_ROUTER_NT
 #undef LM_BATCH_ROUTER
   return 0;
