@@ -74,7 +74,7 @@ using DownMid = TileCfg<192, 256, 4, 2, 2>;
 using DownMidNarrow = TileCfg<192, 128, 4, 2, 2>;  // hidden not a multiple of 256
 using GateHigh = TileCfg<256, 256, 4, 2, 2>;
 using DownHigh = TileCfg<256, 256, 2, 4, 2>;
-constexpr int64_t kLowBelow = 96, kGateHighFrom = 2048, kDownHighFrom = 1024;
+constexpr int64_t kLowBelow = 96, kHighFrom = 1024, kGateHighAlways = 2048;
 
 // The route block of workgroup `lin` (blocks of at most bm routes of one
 // expert, from the offsets lm_moe_align writes: exclusive prefix of the
@@ -444,15 +444,32 @@ int launch_tile(const bf16 *a, const bf16 *w, const int32_t *offsets,
   return LM_OK;
 }
 
+// GateHigh from 1024 routes per expert where its rounds of 256 tiles cost no
+// more than GateMid's of 512: a round of those takes three quarters of the time
+// (a last one of 128 tiles half of it), an expert's last block counts half, and
+// uneven experts add a thirty-second. From 2048 also where they cost a little
+// more, unless GateMid needs one round only. lm_moe_routes, us, GateMid /
+// GateHigh, fragment-order weights: hidden 1024, inter 128, 32 experts, 1600
+// routes per expert 98 / 87, 1400 76 / 78, 2040 112 / 130; hidden 1536, inter
+// 256, 1800 207 / 194, 1400 168 / 175; inter 512, 40 experts, 1600 380 / 370,
+// 1200 300 / 295, 2040 454 / 467; hidden 384, inter 256, 4 experts, 2040 27 / 34.
+bool gate_high(int64_t routes, int64_t cols, int64_t experts) {
+  if (routes < kHighFrom * experts) return false;
+  const int64_t mid = (routes / GateMid::M + experts / 2) * (cols / GateMid::N);
+  const int64_t high = (routes / GateHigh::M + experts / 2) * (cols / GateHigh::N), last = mid % 512;
+  const int64_t mid_time = 3 * (mid / 512) + (last > 128 ? 3 : last > 0 ? 2 : 0);  // quarters of a GateHigh round
+  return mid > 512 && (routes >= kGateHighAlways * experts || 4 * cdiv(high + high / 32, 256) <= mid_time);
+}
+
 }  // namespace
 
 int launch_expert_gemm_gate_up(const bf16 *x, const bf16 *w13, const int32_t *offsets,
                                const int32_t *sorted, int64_t routes, int64_t topk, int64_t hidden,
                                int64_t inter, int64_t experts, bf16 *act, bool packed,
                                bool sorted_act, hipStream_t stream) {
-  auto launch = routes < kLowBelow * experts       ? launch_tile<true, GateLow>
-                : routes < kGateHighFrom * experts ? launch_tile<true, GateMid>
-                                                   : launch_tile<true, GateHigh>;
+  auto launch = routes < kLowBelow * experts                    ? launch_tile<true, GateLow>
+                : gate_high(routes, 2 * inter, experts)        ? launch_tile<true, GateHigh>
+                                                               : launch_tile<true, GateMid>;
   return launch(x, w13, offsets, sorted, routes, topk, hidden, inter, inter, experts, act,
                 packed, sorted_act, stream);
 }
@@ -464,7 +481,7 @@ int launch_expert_gemm_down(const bf16 *act, const bf16 *w2, const int32_t *offs
   const bool wide = hidden % DownMid::N == 0;
   auto launch = routes < kLowBelow * experts       ? launch_tile<false, DownLow>
                 : !wide                            ? launch_tile<false, DownMidNarrow>
-                : routes < kDownHighFrom * experts ? launch_tile<false, DownMid>
+                : routes < kHighFrom * experts ? launch_tile<false, DownMid>
                                                    : launch_tile<false, DownHigh>;
   return launch(act, w2, offsets, sorted, routes, 1, inter, hidden, inter, experts, y, packed,
                 sorted_act, stream);

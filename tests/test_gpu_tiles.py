@@ -281,3 +281,11 @@ def test_linear_dense_narrow_tiles_of_wide_outputs(rows, n, k):
 @torch.inference_mode()
 def test_linear_dense_tile_height_by_padding(rows, n, k):
     test_linear_dense_tiles_match_fp32_product(rows, n, k)
+
+
+@pytest.mark.parametrize("m,h,i,e,k", [
+    (1450, 256, 128, 8, 8), (3000, 256, 256, 16, 8),         # one round of 192 x 128 tiles, more than one
+    (6400, 256, 128, 32, 8), (6200, 384, 128, 32, 8)])       # where 256 x 256 ones take one
+@torch.inference_mode()
+def test_expert_gate_tile_by_rounds(m, h, i, e, k):
+    test_expert_gemm_tiles_match_oracle(m, h, i, e, k)
