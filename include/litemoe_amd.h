@@ -220,9 +220,9 @@ int lm_prefill_attention(const void *q, int64_t qs0, int64_t qs1,
  * summed in selection order. The fp32 accumulation order of the logits
  * depends on the call size: below 1024 tokens a per-token GEMV; from 1024
  * tokens with hidden = 512*{1,2,3,4,6,8} and 16 < experts <= 64, MFMA tiles
- * of 16 tokens (the last tokens % 16 on the GEMV), so a logit can differ by
- * one bf16 ulp between the two, as between any two BLAS orders. The
- * selection is exact given the logits. `renormalize` is a set of flags:
+ * of 16 tokens (the last tokens % 16 on the GEMV; % 32 from hidden 2048), so
+ * a logit can differ by one bf16 ulp between the two, as between any two
+ * BLAS orders. The selection is exact given the logits. `renormalize` is a set of flags:
  * bit 0 (1) softmax over the selection, else over every logit; bit 1 (2)
  * each token's selection written in ascending expert id (weights alongside)
  * instead of descending logit, the order lm_moe_routes_combine_packed sums

@@ -13,18 +13,18 @@
 // the whole buffer.
 //
 // Workgroup = (output column tile, route block). It computes a kTM x kTN
-// fp32 tile (see the tiles below): for gate_up the B tile is kTN/2 gate rows and the kTN/2 up rows
-// of the same j, so silu(g)*u is formed in registers. The waves sit in
-// kWM x kWN, each (kTM/kWM) x (kTN/kWN) as 16 x 16 tiles of
+// fp32 tile (see the tiles below): for gate_up the B tile is kTN/2 gate rows
+// and the kTN/2 up rows of the same j, so silu(g)*u is formed in registers.
+// The waves sit in kWM x kWN, each (kTM/kWM) x (kTN/kWN) as 16 x 16 tiles of
 // v_mfma_f32_16x16x32_bf16.
 //
 // K runs in steps of 64. The next step's A rows (gathered through the route
 // list: each lane's copy has its own address) and B rows are copied from
 // global memory straight into another of the LDS stages
 // (global_load_lds_dwordx4, lds_copy16) while the MFMAs run on the current
-// one. An LDS row is 64 bf16 = 8 chunks of 16 bytes; chunk c of tile row r sits at position
-// c ^ (r & 7), so the 16 rows read by one MFMA fragment load spread over the
-// banks, and each wave instruction fills 1 KB contiguously.
+// one. An LDS row is 64 bf16 = 8 chunks of 16 bytes; chunk c of tile row r sits
+// at position c ^ (r & 7), so the 16 rows read by one MFMA fragment load spread
+// over the banks, and each wave instruction fills 1 KB contiguously.
 //
 // Reference: the expert math of litemoe/ops.py:43-47 (reference_experts) and
 // vLLM fused_experts at litemoe/ep.py:40-41.

@@ -15,16 +15,15 @@
 //
 // Workgroup = kTM x kTN output tile (16 x 64 to 256 x 256, launch_gemm_tiled),
 // kWM x kWN waves, each wave a (kTM/kWM) x (kTN/kWN) block of 16 x 16 MFMA
-// tiles; K runs in steps of 64.
-// The next steps' A and B rows are copied from global memory straight into
-// the other LDS stages (two to four; global_load_lds_dwordx4, no register
-// staging) while the MFMAs run on the current step's stage; one barrier per
-// step. An
-// LDS row is 64 bf16 = 8 chunks of 16 bytes; chunk c of tile row r sits at
-// position c ^ (r & 7), so the 16 rows of one fragment read spread over the
-// banks, and each copy instruction fills 1 KB contiguously. At the cfg 4 QKV
-// shape (46,990 x 1536 -> 2560, one box) the copies take the projection from
-// 472 to 365 us against register staging; at the o_proj shape 261 -> 220 us.
+// tiles; K runs in steps of 64. The next steps' A and B rows are copied from
+// global memory straight into the other LDS stages (two to four;
+// global_load_lds_dwordx4, no register staging) while the MFMAs run on the
+// current step's stage; one barrier per step. An LDS row is 64 bf16 = 8 chunks
+// of 16 bytes; chunk c of tile row r sits at position c ^ (r & 7), so the 16
+// rows of one fragment read spread over the banks, and each copy instruction
+// fills 1 KB contiguously. At the cfg 4 QKV shape (46,990 x 1536 -> 2560, one
+// box) the copies take the projection from 472 to 365 us against register
+// staging; at the o_proj shape 261 -> 220 us.
 // The weights are the MFMA's first operand, so a lane ends with four
 // consecutive output columns of one row. When the output rows allow 16-byte
 // stores, the bf16 tile is staged in the idle LDS stages and each store
@@ -360,8 +359,8 @@ gemm_kernel(const bf16 *__restrict__ a, int64_t lda, const bf16 *__restrict__ w,
     __syncthreads();
     // The rotated q, k, v and the cache rows of a large prefill leave
     // non-temporal: they would push the operand tiles out of the L2s (the
-    // block of 25k tokens at hidden 1024 346 -> 340 us, of 7584 at 1536 165 ->
-    // 162, of 47k unchanged; A/B on one box).
+    // attention block of 25k tokens at hidden 1024 346 -> 340 us, of 7584 at
+    // 1536 165 -> 162, of 47k unchanged; A/B on one box).
     auto store = [&](u32x4 *dst, const u32x4 &word) {
       if constexpr (kRope && kTM >= 192) __builtin_nontemporal_store(word, dst);
       else *dst = word;
@@ -477,10 +476,12 @@ int launch_gemm_cfg(const bf16 *a, int64_t lda, const bf16 *w, int64_t ldw, bf16
   return LM_OK;
 }
 
-// The tile is the smallest whose grid the chip holds at once (its workgroups
-// per CU times 256), so that a launch is one round of workgroups, each with
+// The tile is the smallest whose grid is one round of workgroups, each with
 // little to do, until the operand re-reads of small tiles cost more than idle
-// CUs: below that a launch takes its K loop's latency whatever its size. Up
+// CUs: below that a launch takes its K loop's latency whatever its size. A
+// round is one workgroup per CU for the tiles of 64 columns (three of 64 x 64,
+// two of 128 x 64 fit, but each re-reads the operands more often than the next
+// larger tile), two for 64 x 128 to 192 x 128, one for 256 x 256. Up
 // to 16 rows (the LM head of a few prompts) the weights are all the traffic
 // and the tile's rows are mostly padding. Every tile sums K in the same
 // order, so the choice changes no bits. Measured alone on one box, us

@@ -58,11 +58,12 @@ int launch_align(const int32_t *ids, int64_t routes, int64_t first_expert, int64
                  int64_t scratch_bytes, hipStream_t stream);
 
 // expert_gemm.hip: LDS-tiled MFMA GEMMs over lm_moe_align's route blocks, for
-// prefill-sized route counts (act and y in route order). The line lies just
-// above the scan path's 2048 routes (calls of up to 264 top-8 tokens keep the
-// bits of the block kernels): the MoE block at 290 tokens, 40 experts, hidden
-// 1536 takes 62 us on the GEMMs and 100 on the block kernels (60 and 128 with
-// half of the routes on four experts), at 500 tokens 78 and 134.
+// prefill-sized route counts (act and y in route order). The GEMMs are the
+// faster ones from the scan path's end on (2049 routes); the line lies 64 routes
+// above it, so calls of 257 to 264 top-8 tokens keep the bits that they had
+// from the block kernels, at a price: lm_moe_routes at 40 experts, hidden 1536
+// takes 87 us at 264 tokens and 53 at 265 (92 and 52 with half of the routes on
+// four experts), at 32 experts, hidden 1024 53 and 37.
 constexpr int64_t kExpertGemmMinRoutes = 2113;
 bool expert_gemm_ok(int64_t routes, int64_t hidden, int64_t inter, int64_t experts);
 int launch_expert_gemm_gate_up(const bf16 *x, const bf16 *w13, const int32_t *offsets,
